@@ -60,14 +60,15 @@ __host__ __device__ constexpr int q5h_bit(int e) {
   return 2 * (e >> 3) + ((e >> 1) & 1) + 8 * (((e >> 2) & 1) + 2 * (e & 1));
 }
 
-// Q4_K lane-sliced header (8 x u16 per super-block): d | dmin << 16 from the high
-// nibbles of all eight entries.
+// Q4_K lane-sliced header (8 x u16 per super-block): d | dmin << 16 from the high nibbles of
+// all eight entries.  Nibble 2k sits in byte 1 of word k, nibble 2k + 1 in byte 3: gathered
+// into two words of four bytes each, then merged byte by byte (eight operations; assembling
+// the eight nibbles one by one takes about twenty).
 __device__ __forceinline__ uint32_t q4k_dd(const uint4& h) {
-  const uint32_t w[4] = {h.x, h.y, h.z, h.w};
-  uint32_t dd = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) dd |= ((w[j >> 1] >> (16 * (j & 1) + 12)) & 15u) << (4 * j);
-  return dd;
+  const uint32_t p01 = __builtin_amdgcn_perm(h.y, h.x, 0x07030501u);  // bytes x1, y1, x3, y3
+  const uint32_t p23 = __builtin_amdgcn_perm(h.w, h.z, 0x07030501u);
+  const uint32_t even = __builtin_amdgcn_perm(p23, p01, 0x05040100u), odd = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
+  return ((even >> 4) & 0x0F0F0F0Fu) | (odd & 0xF0F0F0F0u);
 }
 
 // Raw packed bytes of one 32-weight sub-block (what a loader prefetches).

@@ -165,7 +165,7 @@ __global__ void pack_q4_kernel(const uint8_t* __restrict__ src, uint8_t* __restr
 
 // One thread per (row, 32-weight sub-block): 32 outputs.
 template <int QT>
-__global__ void dequant_kernel(PlanePtrs P, int N, int K, void* __restrict__ out, int out_dtype, uint32_t nib) {
+__global__ void dequant_kernel(PlanePtrs P, int N, int K, void* __restrict__ out, int out_dtype) {
   const int nsub = K / 32;
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (size_t)N * nsub) return;
@@ -182,7 +182,7 @@ __global__ void dequant_kernel(PlanePtrs P, int N, int K, void* __restrict__ out
   } else {
     // the routine the MFMA GEMM uses to build its weight operands
     uint4 v[4];
-    dequant_sub_words<QT, X_BF16>(P, K, n, sb, nib, v);
+    dequant_sub_words<QT, X_BF16>(P, K, n, sb, v);
     uint4* dst = (uint4*)((uint16_t*)out + o);
 #pragma unroll
     for (int i = 0; i < 4; ++i) dst[i] = v[i];
@@ -236,17 +236,17 @@ hipError_t launch_dequant(const PackedLayout& L, const uint8_t* packed_dev, void
   const int threads = 256;
   const dim3 grid((unsigned)((total + threads - 1) / threads));
   if (L.qtype == QT_Q4_K)
-    dequant_kernel<QT_Q4_K><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype, 0x0F0F0F0Fu);
+    dequant_kernel<QT_Q4_K><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype);
   else if (L.qtype == QT_Q6_K)
-    dequant_kernel<QT_Q6_K><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype, 0x0F0F0F0Fu);
+    dequant_kernel<QT_Q6_K><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype);
   else if (L.qtype == QT_Q5_K)
-    dequant_kernel<QT_Q5_K><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype, 0x0F0F0F0Fu);
+    dequant_kernel<QT_Q5_K><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype);
   else if (L.qtype == QT_Q4_0)
-    dequant_kernel<QT_Q4_0><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype, 0x0F0F0F0Fu);
+    dequant_kernel<QT_Q4_0><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype);
   else if (L.qtype == QT_Q4_1)
-    dequant_kernel<QT_Q4_1><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype, 0x0F0F0F0Fu);
+    dequant_kernel<QT_Q4_1><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype);
   else
-    dequant_kernel<QT_Q8_0><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype, 0x0F0F0F0Fu);
+    dequant_kernel<QT_Q8_0><<<grid, dim3(threads), 0, s>>>(P, L.N, L.K, out, out_dtype);
   return hipGetLastError();
 }
 

@@ -62,7 +62,6 @@ struct SkinnyParams {
   float* ws;        // K splits over workgroups: fp32 partials, split s at ws + s * ws_split
   size_t ws_split;  // elements per split plane
   int ws_ld;        // workspace row stride (N; 2N for SwiGLU: gate then up columns)
-  uint32_t nib;
   // SwiGLU (narrow kernel only): P2 is the up weight; a slab is 16 rows of both weights
   // (row tile 0 gate, 1 up) and the result swish(gate + bias) * (up + bias2) goes to y
   int swiglu;
@@ -171,10 +170,10 @@ __global__ __launch_bounds__(64 * MAXW) void qgemm_skinny_kernel(SkinnyParams p)
     load_x(kt + 2, std::integral_constant<int, (u + 2) & 3>());
     if constexpr (is_kquant(QT) && (u & 3) == 0) decode_hdr<QT>(hdr[u >> 2], h, sc);
     uint4 w[4];
-    w[0] = dequant_word<QT, XT, 0, true>(raw[u], sc, u & 3, p.nib);
-    w[1] = dequant_word<QT, XT, 1, true>(raw[u], sc, u & 3, p.nib);
-    w[2] = dequant_word<QT, XT, 2, true>(raw[u], sc, u & 3, p.nib);
-    w[3] = dequant_word<QT, XT, 3, true>(raw[u], sc, u & 3, p.nib);
+    w[0] = dequant_word<QT, XT, 0, true>(raw[u], sc, u & 3);
+    w[1] = dequant_word<QT, XT, 1, true>(raw[u], sc, u & 3);
+    w[2] = dequant_word<QT, XT, 2, true>(raw[u], sc, u & 3);
+    w[3] = dequant_word<QT, XT, 3, true>(raw[u], sc, u & 3);
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
@@ -282,7 +281,7 @@ __device__ __forceinline__ void decode_hdr16(const Hdr<QT>& h, int j, Scales<QT>
   const uint32_t w[4] = {h.h[0], h.h[1], h.h[2], h.h[3]};
   if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
     const uint32_t dd = q4k_dd(make_uint4(w[0], w[1], w[2], w[3]));
-    const float d = f16_bits_to_f32(dd & 0xffffu), dmin = f16_bits_to_f32(dd >> 16);
+    const float d = f16_bits_to_f32(dd & 0xffffu) * SUB24, dmin = f16_bits_to_f32(dd >> 16);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const uint32_t v = w[2 * q + (j >> 1)];
@@ -291,7 +290,7 @@ __device__ __forceinline__ void decode_hdr16(const Hdr<QT>& h, int j, Scales<QT>
       s.b[q] = -(dmin * (float)(f >> 6));
     }
   } else if constexpr (QT == QT_Q6_K) {
-    const float d = f16_bits_to_f32(h.d & 0xffffu);
+    const float d = f16_bits_to_f32(h.d & 0xffffu) * SUB24;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const uint32_t v0 = w[2 * q + (j >> 1)];
@@ -477,10 +476,10 @@ __global__ __launch_bounds__(64 * MAXW) void qgemm_skinny16_kernel(SkinnyParams 
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       uint4 w[4];
-      w[0] = dequant_word<QT, XT, 0, true>(raw[ru][t], sc[t], u & 1, p.nib);
-      w[1] = dequant_word<QT, XT, 1, true>(raw[ru][t], sc[t], u & 1, p.nib);
-      w[2] = dequant_word<QT, XT, 2, true>(raw[ru][t], sc[t], u & 1, p.nib);
-      w[3] = dequant_word<QT, XT, 3, true>(raw[ru][t], sc[t], u & 1, p.nib);
+      w[0] = dequant_word<QT, XT, 0, true>(raw[ru][t], sc[t], u & 1);
+      w[1] = dequant_word<QT, XT, 1, true>(raw[ru][t], sc[t], u & 1);
+      w[2] = dequant_word<QT, XT, 2, true>(raw[ru][t], sc[t], u & 1);
+      w[3] = dequant_word<QT, XT, 3, true>(raw[ru][t], sc[t], u & 1);
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
@@ -768,7 +767,6 @@ hipError_t launch_skinny(const RunArgs& a, hipStream_t s) {
   sp.K = a.L.K;
   sp.bias_dtype = a.bias_dtype;
   sp.y_dtype = a.y_dtype;
-  sp.nib = 0x0F0F0F0Fu;
   sp.ws = (float*)a.ws;
   sp.swiglu = 0;
   sp.P2 = sp.P;
@@ -804,7 +802,6 @@ SkinnyParams swiglu_params(const RunArgs& gate, const RunArgs& up) {
   sp.K = gate.L.K;
   sp.bias_dtype = gate.bias_dtype;
   sp.y_dtype = gate.y_dtype;
-  sp.nib = 0x0F0F0F0Fu;
   sp.ws = (float*)gate.ws;
   sp.swiglu = 1;
   return sp;

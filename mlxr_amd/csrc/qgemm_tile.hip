@@ -247,7 +247,6 @@ hipError_t launch_mfma(const RunArgs& a, hipStream_t s) {
     tp.M = M;
     tp.K = K;
     tp.x = a.x;
-    tp.nib = 0x0F0F0F0Fu;
     tp.kps = sp.kps;
     tp.ws = (float*)a.ws;
     tp.ws_split = (size_t)M * (size_t)N;
@@ -279,7 +278,6 @@ hipError_t launch_mfma(const RunArgs& a, hipStream_t s) {
       tp.M = std::min(Mc, M - mc);
       tp.K = K;
       tp.x = (const uint8_t*)a.x + (size_t)mc * K * 2;
-      tp.nib = 0x0F0F0F0Fu;
       tp.kps = (K + TK - 1) / TK;
       tp.ws = nullptr;
       tp.ws_split = 0;
@@ -349,7 +347,6 @@ hipError_t launch_mfma_grouped(const RunArgs* const* items, int n, void* ws, siz
   tp.M = M;
   tp.K = K;
   tp.x = a.x;
-  tp.nib = 0x0F0F0F0Fu;
   tp.kps = sp.S > 1 ? sp.kps : (K + TK - 1) / TK;
   tp.ws = sp.S > 1 ? (float*)ws : nullptr;
   tp.ws_split = (size_t)M * (size_t)cols;
@@ -423,7 +420,6 @@ hipError_t launch_mfma_swiglu(const RunArgs& gate, const RunArgs& up, void* ws, 
   tp.M = M;
   tp.K = K;
   tp.x = gate.x;
-  tp.nib = 0x0F0F0F0Fu;
   tp.kps = split ? sp.kps : (K + TK - 1) / TK;
   tp.ws = split ? (float*)ws : nullptr;
   tp.ws_split = (size_t)M * (size_t)N * 2u;

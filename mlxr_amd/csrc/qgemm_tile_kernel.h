@@ -85,7 +85,6 @@ struct TileParams {
   float* ws;        // split-K: fp32 partials, split s at ws + s * ws_split, rows of ws_ld
   size_t ws_split;  // elements per split plane
   int ws_ld;        // workspace row stride (the launch's total N)
-  uint32_t nib;     // 0x0F0F0F0F, passed at run time (keeps the byte converts)
   int ngroups;
   // SwiGLU (gate = g[0], up = g[1], same shape): a tile is 128 output columns; wavefront
   // w's two 32-column accumulator blocks are gate and up of the same 32 columns, and the
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_tile_kernel(TileParams p) {
   sfor<4>([&](auto KK) {
     constexpr int kk = decltype(KK)::value;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bf[j][kk] = dequant_word<QT, XT, kk, true>(raw[0][j], sc[j], 0, p.nib);
+    for (int j = 0; j < 2; ++j) bf[j][kk] = dequant_word<QT, XT, kk, true>(raw[0][j], sc[j], 0);
   });
   // stage 0 complete (every wavefront's DMA of it) before its first fragments are read
   vm_wait<2 * MI + rops(PD - 2) + rops(PD - 1)>();
@@ -365,8 +364,8 @@ __global__ __launch_bounds__(256, 1) void qgemm_tile_kernel(TileParams p) {
         constexpr int k = decltype(TK_)::value;
         if constexpr ((k * SPS) / 10 == ts) {
           constexpr int jw = k / 5, kq = k % 5;
-          if constexpr (kq == 0) word_prelude<QT, kk, true>(raw[un][jw], sc[jw], un & 3, p.nib, wt[jw]);
-          else nw[jw][kq - 1] = word_quarter<QT, XT, kk, kq - 1, true>(wt[jw], p.nib);
+          if constexpr (kq == 0) word_prelude<QT, kk, true>(raw[un][jw], sc[jw], un & 3, wt[jw]);
+          else nw[jw][kq - 1] = word_quarter<QT, XT, kk, kq - 1, true>(wt[jw]);
         }
       });
       if constexpr (ts == SPS - 1) {
