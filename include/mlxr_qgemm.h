@@ -268,12 +268,11 @@ int mlxr_qgemm_mlp_status(void* workspace_dev, void* stream);
  * bound in ticks of the 100 MHz real-time counter (default 0.2 s; 0 restores it), lowered
  * by tests to exercise the timeout path.  mlxr_qgemm_test_force_skinny(1): every call of the
  * MFMA family (M > 4, or MLXR_PATH_MFMA) runs the skinny kernel, at any M, until called
- * with 0; tests use it to reach the skinny kernel's 64-row M blocks at shapes the automatic
- * choice gives to the tiled kernel.  mlxr_qgemm_test_skinny_stage(0): the narrow skinny
- * kernel reads its activations from global memory at every step instead of staging them in
- * LDS once (its mode at M <= 16 when the stages fit; 1 restores it; 2 prefers the mode where
- * two slabs share their stages wherever it fits); tests use it to check every mode against
- * the oracle.  All are process-wide (atomics). */
+ * with 0; tests use it to reach the skinny kernel's blocks of M at shapes the automatic
+ * choice gives to the tiled kernel.  mlxr_qgemm_test_skinny_stage: weight tiles a wavefront of
+ * the skinny kernel takes: 0 one, 2 two, 3 and above four (SwiGLU: two, two, four), 1 restores
+ * the choice by shape; tests use it to check every variant against the oracle.
+ * All are process-wide (atomics). */
 int mlxr_qgemm_test_set_operand_limit(size_t bytes);
 int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks);
 int mlxr_qgemm_test_force_skinny(int on);

@@ -480,7 +480,7 @@ namespace {
 int swiglu_kind(const mlxr::RunArgs& a) {
   if (a.M <= kGemvMaxM && gemv_auto(a.M, a.L) && mlxr::gemv_groupable(a)) return 0;
   if (!mlxr::mfma_groupable(a)) return 3;
-  return mlxr::skinny_swiglu_ok(a.M) ? 1 : 2;
+  return a.M <= kSkinnyOnlyMaxM ? 1 : 2;
 }
 }  // namespace
 
@@ -703,7 +703,7 @@ int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks) {
 }
 
 int mlxr_qgemm_test_skinny_stage(int on) {
-  mlxr::g_skinny_stage.store(on <= 0 ? 0 : on >= 2 ? 2 : 1, std::memory_order_relaxed);
+  mlxr::g_skinny_stage.store(on <= 0 ? 0 : on >= 3 ? 4 : on, std::memory_order_relaxed);
   return MLXR_OK;
 }
 

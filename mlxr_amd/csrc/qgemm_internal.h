@@ -74,25 +74,26 @@ int device_cu_count();
 // device's opt-in maximum, at most 160 KiB (gfx950), queried once per device.
 size_t device_lds_limit();
 
-// Skinny MFMA GEMM for M <= 64 (qgemm_skinny.hip), weights streamed once.  With a.ws,
-// shapes with fewer 32-row slabs than CUs also split K over workgroups.
+// Skinny MFMA GEMM (qgemm_skinny.hip): any M in blocks of up to 32 rows, the weights streamed
+// once per block.  It takes no workspace.
 hipError_t launch_skinny(const RunArgs& a, hipStream_t s);
-// Whether the narrow skinny kernel stages its activations in LDS where they fit (default 1;
-// test hook mlxr_qgemm_test_skinny_stage).
+// Up to 4 weights of one quant type and K sharing x and M in one launch (skinny_fits each);
+// equal to separate launches bit for bit.
+hipError_t launch_skinny_grouped(const RunArgs* const* items, int n, hipStream_t s);
+// How many weight tiles a wavefront of the skinny kernel takes: 1 chosen by shape (default),
+// 0 one, 2 two, 4 four (test hook mlxr_qgemm_test_skinny_stage).
 extern std::atomic<int> g_skinny_stage;
 // Whether every operand of a is below operand_limit() (else: launch_mfma, which chunks).
 bool skinny_fits(const RunArgs& a);
-// Workspace bytes launch_skinny would use (0: no split).
+// Workspace bytes reported for shapes of the skinny kernel (0: none).
 size_t skinny_workspace_bytes(int M, int N, int K, int qtype);
-// Estimated time of launch_skinny for M > 32 (64-row blocks of M over a second grid
-// dimension) and of launch_mfma with a workspace of ws_bytes, in microseconds.
+// Estimates in microseconds that decide which kernel's workspace size is reported for 32 < M
+// <= 256: a skinny kernel in 64-row blocks, and launch_mfma with a workspace of ws_bytes.
 double skinny_mb_est_us(int M, int N, int K);
 double mfma_est_us(int M, int N, int K, int qtype, size_t ws_bytes);
 // SwiGLU, h = swish(x.gate^T + bias_g) * (x.up^T + bias_u) into gate.y, with gate and up
 // of one type and shape; gate.ws / ws (may be null) holds split-K partials.
-// Narrow skinny kernel (M <= 32, skinny_swiglu_ok) and tiled kernel (any M; operands
-// below 2 GiB, mfma_groupable; no biases).
-bool skinny_swiglu_ok(int M);
+// Skinny kernel and tiled kernel (any M; operands below 2 GiB, mfma_groupable; no biases).
 hipError_t launch_skinny_swiglu(const RunArgs& gate, const RunArgs& up, hipStream_t s);
 size_t skinny_swiglu_workspace_bytes(int M, int N, int K);
 hipError_t launch_mfma_swiglu(const RunArgs& gate, const RunArgs& up, void* ws, size_t ws_bytes, hipStream_t s);

@@ -216,6 +216,13 @@ __device__ __forceinline__ void word_prelude(const Raw<QT>& r, const Scales<QT>&
   t.a4 = t.a * 0.0625f;
 }
 
+// v shifted so that bit `from` comes to bit `at`.
+template <int from, int at>
+__device__ __forceinline__ uint32_t move_bits(uint32_t v) {
+  if constexpr (at >= from) return v << (at - from);
+  else return v >> (from - at);
+}
+
 // The codes of pair qq of word kk as subnormal halves.  Pairs 0 and 2 take the low nibbles
 // of their bytes (bits 0 and 16), pairs 1 and 3 the high ones in place (bits 4 and 20), with
 // their high bits on top.
@@ -225,12 +232,12 @@ __device__ __forceinline__ uint32_t pair_codes(const WordTmp<QT>& t) {
   if constexpr (QT == QT_Q5_K) {
     // the fifth bits of word kk's pairs sit at bits 2kk, 2kk + 1, 2kk + 8, 2kk + 9 of each half
     constexpr int from = 2 * kk + (qq & 1) + 4 * (qq & 2), at = (qq & 1) ? 8 : 4;
-    const uint32_t h = at >= from ? t.x << (at - from) : t.x >> (from - at);
+    const uint32_t h = move_bits<from, at>(t.x);
     return n | (h & ((qq & 1) ? 0x01000100u : 0x00100010u));
   } else if constexpr (QT == QT_Q6_K) {
     // the two high bits of pair qq sit at bits 2qq, 2qq + 1 of each half
     constexpr int from = 2 * qq, at = (qq & 1) ? 8 : 4;
-    const uint32_t h = at >= from ? t.x << (at - from) : t.x >> (from - at);
+    const uint32_t h = move_bits<from, at>(t.x);
     return n | (h & ((qq & 1) ? 0x03000300u : 0x00300030u));
   } else {
     return n;

@@ -439,13 +439,12 @@ def test_set_mlp_spin_limit(ticks):
 
 
 def test_force_skinny(on):
-    """Test hook: send every MFMA-family call to the skinny kernel (any M, in 64-row blocks
-    of M above 32) while on."""
+    """Test hook: send every MFMA-family call to the skinny kernel (any M, in blocks
+    of M) while on."""
     _check(lib().mlxr_qgemm_test_force_skinny(1 if on else 0))
 
 
 def test_skinny_stage(mode):
-    """Test hook: whether the narrow skinny kernel stages its activations in LDS where they
-    fit (True / 1, the default); False / 0: it reads them from global memory at every step;
-    2: two slabs per workgroup share their stages wherever that fits."""
+    """Test hook: weight tiles a wavefront of the skinny kernel takes: 0 (False) one, 2 two,
+    3 and above four (SwiGLU: two, two, four); 1 (True, the default) chooses by shape."""
     _check(lib().mlxr_qgemm_test_skinny_stage(int(mode)))

@@ -527,6 +527,38 @@ def test_skinny_staged_activations_match_oracle(cuda, qt, M, N, K, path, ydt):
     assert orc.rel_err(ys[1].float().cpu().numpy(), ref) <= (5e-3 if ydt != "f32" else 3e-5)
 
 
+@pytest.mark.parametrize("qt,M,N,K", [(Q4K, 5, 63, 256), (Q4K, 8, 65, 2048), (Q6K, 9, 130, 2304), (Q5K, 16, 17, 4352),
+                                      (Q80, 17, 33, 32), (Q41, 32, 100, 2080), (Q40, 33, 129, 4064), (Q6K, 64, 47, 512),
+                                      (Q4K, 65, 1, 2304), (Q80, 100, 66, 2048), (Q5K, 31, 64, 256), (Q40, 7, 16, 96)])
+def test_skinny_tile_counts_match_oracle(cuda, qt, M, N, K):
+    """One, two and four weight tiles per wavefront of the skinny kernel, at the edges of its
+    8-, 16- and 32-row blocks, of its 16- to 64-row slabs and of K (one block; less or more than
+    the 8 wavefronts' super-blocks): the same bits, and the oracle within the error of fp32
+    sums.  A product takes part in at most 32 additions of its MFMA, 8 MFMAs of its super-block,
+    one addition per 2048 of K and 8 over the wavefronts; each is within 2^-23 (whether it
+    rounds or truncates) of partial sums that the sum of |w x| bounds."""
+    import torch
+    w, pw = _packed(torch, qt, N, K, 411 + M, cuda)
+    x, xf = _act(torch, M, K, mx.BF16, 421 + M, cuda)
+    ys = {}
+    try:
+        mx.qgemm.test_force_skinny(True)
+        for mode in (1, 0, 2, 4):
+            mx.qgemm.test_skinny_stage(mode)
+            ys[mode] = mx.q_gemm_dequant(x, pw, M, N, K, qt, out_dtype=torch.float32, path=mx.PATH_MFMA)
+    finally:
+        mx.qgemm.test_skinny_stage(1)
+        mx.qgemm.test_force_skinny(False)
+    torch.cuda.synchronize()
+    for mode in (0, 2, 4):
+        assert torch.equal(ys[mode], ys[1]), mode
+    ref = orc.gemm_f64(int(qt), M, N, K, w, xf, w_to_bf16=True).astype(np.float64)
+    wabs = np.abs(orc.dequant(int(qt), N, K, w).reshape(N, K).astype(np.float64)) * (1 + 2.0**-8)
+    bound = np.abs(xf.astype(np.float64)) @ wabs.T * (32 + 8 + K // 2048 + 1 + 8) * 2.0**-23
+    d = np.abs(ys[1].cpu().numpy().astype(np.float64) - ref)
+    assert (d <= bound + 2.0**-24 * np.abs(ref)).all(), (d - bound).max()
+
+
 @pytest.mark.parametrize("qt,M", [(Q4K, 8), (Q80, 5), (Q6K, 3)])
 def test_skinny_staged_f16_activations_match_oracle(cuda, qt, M):
     """fp16 activations (the fp16 MFMA, fp16-rounded weights) through the staged narrow
