@@ -184,9 +184,9 @@ typedef struct mlxr_qgemm_item {
 /* y_i[M, N_i] = X[M, K] . W_i[N_i, K]^T (+ bias_i) for `count` weights that read the same
  * activations -- the projections of one input, e.g. q/k/v or gate/up of a decoder layer.
  * Every item must have the same K.  Items of one quant type run up to four per launch
- * where the kernel allows it: the GEMV at M <= 4 (X staged once) and the tiled MFMA GEMM
- * at M > 64 (tile columns of the weights side by side); other items run as
- * mlxr_qgemm_run(..., MLXR_PATH_AUTO).  Results equal count separate mlxr_qgemm_run calls
+ * where the kernel allows it: the GEMV at M <= 4 (X staged once), the skinny MFMA kernel to
+ * M = 64 and the tiled MFMA GEMM above (slabs or tile columns of the weights side by side); other
+ * items run as mlxr_qgemm_run(..., MLXR_PATH_AUTO).  Results equal count separate mlxr_qgemm_run calls
  * bit for bit, with one exception at M <= 4: an item whose single call the automatic path
  * gives the skinny MFMA kernel (mlxr_qgemm_auto_path) stays in the GEMV launch unless its
  * weight is very large (N*K >= 128 Mi elements), and then equals its single call with
@@ -196,9 +196,10 @@ typedef struct mlxr_qgemm_item {
 int mlxr_qgemm_run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,
                            void* stream);
 /* mlxr_qgemm_run_grouped with a caller-owned device workspace (NULL or too small = as
- * mlxr_qgemm_run_grouped).  With it the tiled launches also serve 32 < M <= 64 and split K
- * over the concatenated N of their weights when their tiles cannot fill the device, and
- * single items run as mlxr_qgemm_run_ws.  Results then differ from separate calls only in
+ * mlxr_qgemm_run_grouped).  With it, launches at 32 < M <= 256 go to the skinny or the
+ * tiled kernel, whichever is estimated faster for the weights together, the tiled launches split
+ * K over the concatenated N of their weights when their tiles cannot fill the device, and single
+ * items run as mlxr_qgemm_run_ws.  Results then differ from separate calls only in
  * fp32 summation order (within the matmul tolerance) and are deterministic for a given
  * (items, M, workspace size).  Same workspace rules as mlxr_qgemm_run_ws. */
 int mlxr_qgemm_run_grouped_ws(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,

@@ -36,27 +36,25 @@ bool gemv_auto(int M, const mlxr::PackedLayout& L) {
   if (M == 4 && (long)L.N * (long)L.K >= (48L << 20) && L.qtype != mlxr::QT_Q6_K) return false;
   return true;
 }
-// Up to this M the skinny kernel serves every MFMA call (measured on MI355X, Llama-3-8B
-// FFN shapes: at M = 32 its 16x16x32 variant is ahead of the tiled GEMM with 64-row tiles
-// and split-K, gate 26.9 vs 29.0 us and down 26.7 vs 29.7 us; at M = 64 the tiled one,
-// gate 28.3 vs 42.7 us).
+// Up to this M the skinny kernel serves every MFMA call (measured on MI355X, Q4_K, us, skinny /
+// tiled at M = 33, where the skinny kernel begins a second block of rows: 1024 x 4096 7.1 /
+// 10.6, 4096 x 4096 10.2 / 15.0, 4096 x 14336 24.1 / 24.9, 14336 x 4096 25.9 / 24.1; at M = 24
+// the last takes it 15.7).
 constexpr int kSkinnyOnlyMaxM = 32;
 int skinny_only_max_m() { return kSkinnyOnlyMaxM; }
-// Up to this M a single call chooses between the skinny kernel (in 64-row blocks of M)
-// and the tiled one by their estimated times: on MI355X the skinny one wins for narrow
-// weights, e.g. Llama-3-8B k/v at M = 128: 12.3 against 18.6 us.
+// Up to this M a call chooses between the skinny kernel (in blocks of 32 rows) and the tiled
+// one by their estimated times: on MI355X the skinny one is ahead for narrow weights, e.g.
+// Llama-3-8B k/v at M = 256 9.2 against 17.5 us.
 constexpr int kSkinnyMaxM = 256;
 
-// For skinny_only_max_m() < M <= kSkinnyMaxM: whether the skinny kernel serves a call that
-// has the workspace the library asks for (ws) or none.  Without one the skinny kernel
-// takes M <= 64 and the tiled one (unsplit) larger M.
-bool skinny_mid(int M, const mlxr::PackedLayout& L, bool ws) {
-  if (!ws) return M <= 64;
+// For skinny_only_max_m() < M <= kSkinnyMaxM: the kernel whose workspace size is reported, the
+// skinny one (true) or the tiled one.  Callers size their buffers by it, and
+// mlxr_qgemm_run_noalloc takes or refuses a call by them.
+bool mid_sized_skinny(int M, const mlxr::PackedLayout& L) {
   return mlxr::skinny_mb_est_us(M, L.N, L.K) < mlxr::mfma_est_us(M, L.N, L.K, L.qtype, ~(size_t)0);
 }
-// The workspace size for those M: that of the kernel skinny_mid picks with one.
 void mid_workspace(int M, const mlxr::PackedLayout& L, size_t* bytes) {
-  *bytes = skinny_mid(M, L, true) ? mlxr::skinny_workspace_bytes(M, L.N, L.K, L.qtype)
+  *bytes = mid_sized_skinny(M, L) ? mlxr::skinny_workspace_bytes(M, L.N, L.K, L.qtype)
                                   : mlxr::mfma_workspace_bytes(M, L.N, L.K);
 }
 std::atomic<int> g_force_skinny{0};
@@ -297,7 +295,7 @@ int mlxr_qgemm_run_ws(int qtype, int N, int K, int group_size, const void* packe
   a.ws = workspace_dev;
   a.ws_bytes = workspace_dev ? workspace_bytes : 0;
   // GEMV (no MFMA) for decode (gemv_auto); MFMA kernels otherwise: the skinny one up to
-  // M = 32, then up to M = 256 the skinny or the tiled one (skinny_mid), the tiled one above
+  // M = 32, then up to M = 256 the skinny or the tiled one, the tiled one above
   // (MLXR_PATH_GEMV / MLXR_PATH_MFMA force the family)
   const bool gemv = path == MLXR_PATH_GEMV || (path == MLXR_PATH_AUTO && gemv_auto(M, a.L));
   // the skinny kernels address operands with 32-bit offsets; the tiled launcher splits
@@ -317,7 +315,14 @@ int mlxr_qgemm_run_ws(int qtype, int N, int K, int group_size, const void* packe
       a.ws = nullptr;
       a.ws_bytes = 0;
     }
-    skinny = mlxr::skinny_fits(a) && skinny_mid(M, a.L, ws_ok);
+    // with it, the tiled kernel runs where its size was reported and it is estimated to be
+    // ahead (4096 x 4096 Q4_K, us, tiled / skinny: M = 64 18.1 / 10.7, M = 128 23.7 / 14.4, M =
+    // 256 26.9 / 24.6; 14336 x 4096: M = 64 25.9 / 26.2, M = 128 33.4 / 47.6); without, the
+    // skinny one takes M <= 64 and the tiled one (unsplit) larger M
+    const mlxr::RunArgs* one[1] = {&a};
+    skinny = mlxr::skinny_fits(a) &&
+             (ws_ok ? mid_sized_skinny(M, a.L) || mlxr::skinny_est_us(one, 1) < mlxr::mfma_est_us(M, N, K, qtype, ~(size_t)0)
+                    : M <= 64);
   }
   hipError_t e;
   if (gemv) e = mlxr::launch_gemv(a, (hipStream_t)stream);
@@ -341,27 +346,33 @@ bool grouped_gemv(int M, const mlxr::RunArgs& a) {
   return mlxr::gemv_groupable(a) && (gemv_auto(M, a.L) || (long)a.L.N * (long)a.L.K < (128L << 20));
 }
 
-// How a grouped call runs its items: launches of several items (GEMV at M <= 4, tiled MFMA
-// where the tiled kernel serves the call) and single calls for the rest.
+// How a grouped call runs its items: launches of several items (GEMV at M <= 4, skinny or tiled
+// MFMA) and single calls for the rest.
+enum BatchKind { kSingle, kGroupedGemv, kGroupedTiled, kGroupedSkinny };
 struct Batch {
-  int kind;  // 0 single call, 1 grouped GEMV, 2 grouped tiled MFMA
+  BatchKind kind;
   int idx[4];
   int n;
 };
-std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool with_ws) {
+// The batches a workspace is sized for: those of `sized`, where only GEMV and tiled launches
+// (with_ws, or M > 64) take several items.
+std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool with_ws, bool sized) {
   const int count = (int)a.size();
   const bool tiled = M > 64 || (M > skinny_only_max_m() && with_ws);
+  auto kind_of = [&](const mlxr::RunArgs& r) {
+    if (M <= kGemvMaxM && grouped_gemv(M, r)) return kGroupedGemv;
+    if (tiled) return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
+    return !sized && !gemv_auto(M, r.L) && mlxr::skinny_fits(r) ? kGroupedSkinny : kSingle;
+  };
   std::vector<bool> done((size_t)count, false);
   std::vector<Batch> out;
   for (int i = 0; i < count; ++i) {
     if (done[i]) continue;
-    const int kind = (M <= kGemvMaxM && grouped_gemv(M, a[i])) ? 1 : (tiled && mlxr::mfma_groupable(a[i])) ? 2 : 0;
-    Batch bt{kind, {i, 0, 0, 0}, 1};
+    Batch bt{kind_of(a[i]), {i, 0, 0, 0}, 1};
     done[i] = true;
-    if (kind != 0) {
+    if (bt.kind != kSingle) {
       for (int j = i + 1; j < count && bt.n < 4; ++j) {
-        if (done[j] || a[j].L.qtype != a[i].L.qtype) continue;
-        if (kind == 1 ? !grouped_gemv(M, a[j]) : !mlxr::mfma_groupable(a[j])) continue;
+        if (done[j] || a[j].L.qtype != a[i].L.qtype || kind_of(a[j]) != bt.kind) continue;
         bt.idx[bt.n++] = j;
         done[j] = true;
       }
@@ -369,6 +380,20 @@ std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool
     out.push_back(bt);
   }
   return out;
+}
+
+// Whether a tiled batch of a call that has a workspace runs on the skinny kernel instead: by the
+// estimates of a single weight with the batch's columns (Llama-3-8B q,k,v Q4_K at M = 64, us,
+// tiled / skinny: 23.0 / 14.6).
+bool batch_skinny(const mlxr::RunArgs* const* items, int n, int M, size_t ws_bytes) {
+  if (M > kSkinnyMaxM) return false;
+  int cols = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!mlxr::skinny_fits(*items[i])) return false;
+    if (items[i]->L.N > INT32_MAX / 4) return false;
+    cols += items[i]->L.N;
+  }
+  return mlxr::skinny_est_us(items, n) < mlxr::mfma_est_us(M, cols, items[0]->L.K, items[0]->L.qtype, ws_bytes);
 }
 
 // Validates the items (each exactly as a single call) and fills their run arguments.
@@ -412,13 +437,16 @@ int run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int 
   int rc = grouped_args(count, items, x_dev, x_dtype, M, true, stream, a);
   if (rc || count == 0 || M == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
-  for (const Batch& bt : plan_batches(a, M, ws != nullptr)) {
+  for (const Batch& bt : plan_batches(a, M, ws != nullptr, false)) {
     const mlxr::RunArgs* batch[4];
     for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
-    if (bt.kind == 1) {
+    if (bt.kind == kGroupedGemv) {
       const hipError_t e = mlxr::launch_gemv_grouped(batch, bt.n, s);
       if (e != hipSuccess) return hip_fail(e, "grouped gemv launch");
-    } else if (bt.kind == 2) {
+    } else if (bt.kind == kGroupedSkinny || (bt.kind == kGroupedTiled && ws && batch_skinny(batch, bt.n, M, ws_bytes))) {
+      const hipError_t e = mlxr::launch_skinny_grouped(batch, bt.n, s);
+      if (e != hipSuccess) return hip_fail(e, "grouped skinny launch");
+    } else if (bt.kind == kGroupedTiled) {
       const hipError_t e = mlxr::launch_mfma_grouped(batch, bt.n, ws, ws ? ws_bytes : 0, s);
       if (e != hipSuccess) return hip_fail(e, "grouped mfma launch");
     } else {
@@ -452,13 +480,13 @@ int mlxr_qgemm_grouped_workspace_size(int count, const mlxr_qgemm_item* items, i
   if (rc) return rc;
   size_t need = 0;
   if (count > 0 && M > 0) {
-    for (const Batch& bt : plan_batches(a, M, true)) {
+    for (const Batch& bt : plan_batches(a, M, true, true)) {
       const mlxr::RunArgs* batch[4];
       for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
       size_t b = 0;
-      if (bt.kind == 2) {
+      if (bt.kind == kGroupedTiled) {
         b = mlxr::mfma_grouped_workspace_bytes(batch, bt.n);
-      } else if (bt.kind == 0) {
+      } else if (bt.kind == kSingle) {
         const mlxr_qgemm_item& it = items[bt.idx[0]];
         rc = mlxr_qgemm_workspace_size(it.qtype, it.N, it.K, M, &b);
         if (rc) return rc;

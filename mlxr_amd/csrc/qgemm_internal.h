@@ -80,6 +80,8 @@ hipError_t launch_skinny(const RunArgs& a, hipStream_t s);
 // Up to 4 weights of one quant type and K sharing x and M in one launch (skinny_fits each);
 // equal to separate launches bit for bit.
 hipError_t launch_skinny_grouped(const RunArgs* const* items, int n, hipStream_t s);
+// Estimated time of such a launch for M > 32, in microseconds.
+double skinny_est_us(const RunArgs* const* items, int n);
 // How many weight tiles a wavefront of the skinny kernel takes: 1 chosen by shape (default),
 // 0 one, 2 two, 4 four (test hook mlxr_qgemm_test_skinny_stage).
 extern std::atomic<int> g_skinny_stage;

@@ -519,24 +519,26 @@ hipError_t launch_rt(const SkinnyParams& sp, hipStream_t s) {
 // 4096 at M = 8 14.2 / 13.5 / 12.6, at M = 24 22.2 / 18.3 / 15.3; 8192 x 8192 at M = 13 16.5 /
 // 14.9 / 19.6; 4096 x 4096 at M = 8 6.0 / 7.9 / 10.8; 2 x 28672 x 8192 SwiGLU at M = 13 86 (two)
 // / 78 (four).
-int tiles_for(const SkinnyParams& sp) {
+// Items of n weights (SwiGLU: gate's rows) at rt tiles per wavefront.
+long items_of(const int* N, int n, int M, bool swiglu, int rt) {
+  const int rows = swiglu ? 8 * rt : 16 * rt;
+  long slabs = 0;
+  for (int i = 0; i < n; ++i) slabs += (N[i] + rows - 1) / rows;
+  return slabs * ((M + 31) / 32);
+}
+int tiles_for(const int* N, int n, int M, bool swiglu) {
   const int mode = g_skinny_stage.load(std::memory_order_relaxed);  // 1: by shape; 0, 2, 4: one, two, four tiles
-  const int mblocks = (sp.M + 31) / 32;
-  auto items = [&](int rt) {
-    long n = 0;
-    const int rows = sp.swiglu ? 8 * rt : 16 * rt;
-    for (int i = 0; i < (sp.swiglu ? 1 : sp.ngroups); ++i) n += (sp.g[i].N + rows - 1) / rows;
-    return n * mblocks;
-  };
   const long want = (long)device_cu_count() * 3 / 4;
-  if (sp.swiglu) return mode == 4 || (mode == 1 && items(4) >= want) ? 4 : 2;
+  if (swiglu) return mode == 4 || (mode == 1 && items_of(N, n, M, true, 4) >= want) ? 4 : 2;
   if (mode != 1) return mode == 0 ? 1 : mode;
-  return items(4) >= want ? 4 : items(2) >= want ? 2 : 1;
+  return items_of(N, n, M, false, 4) >= want ? 4 : items_of(N, n, M, false, 2) >= want ? 2 : 1;
 }
 
 template <int QT, int XT>
 hipError_t launch_s(const SkinnyParams& sp, hipStream_t s) {
-  const int rt = tiles_for(sp);
+  int N[MAX_SG];
+  for (int i = 0; i < sp.ngroups; ++i) N[i] = sp.g[i].N;
+  const int rt = tiles_for(N, sp.swiglu ? 1 : sp.ngroups, sp.M, sp.swiglu != 0);
   if (sp.swiglu) return rt == 4 ? launch_rt<QT, XT, 4, 1, true>(sp, s) : launch_rt<QT, XT, 2, 2, true>(sp, s);
   return rt == 4   ? launch_rt<QT, XT, 4, 1, false>(sp, s)
          : rt == 2 ? launch_rt<QT, XT, 2, 2, false>(sp, s)
@@ -641,6 +643,22 @@ hipError_t launch_skinny_swiglu(const RunArgs& gate, const RunArgs& up, hipStrea
   u.y = gate.y;
   const RunArgs* items[2] = {&gate, &u};
   return launch_any(items, 2, true, s);
+}
+
+// Rounds of items over the CUs (one workgroup each at 32 rows), each as long as its K (ns per
+// element at one, two, four tiles; measured on MI355X, Q4_K, us, estimate / time: 8192 x 8192 at
+// M = 64 24.5 / 24.9, at M = 96 45.0 / 45.0; 14336 x 4096 at M = 96 34.7 / 36.3; 4096 x 14336 at
+// M = 128 39.8 / 37.5; 4096 x 4096 at M = 33 10.6 / 10.2, at M = 256 24.5 / 24.6), the other types
+// by their dequantization (4096 x 14336 Q6_K at M = 64 33.8 / 33.6).
+double skinny_est_us(const RunArgs* const* items, int n) {
+  const RunArgs& a = *items[0];
+  int N[MAX_SG];
+  for (int i = 0; i < n; ++i) N[i] = items[i]->L.N;
+  const int rt = tiles_for(N, n, a.M, false);
+  const int cus = device_cu_count();
+  const long rounds = (items_of(N, n, a.M, false, rt) + cus - 1) / cus;
+  const double qf = a.L.qtype == QT_Q6_K ? 1.3 : a.L.qtype == QT_Q5_K ? 1.16 : a.L.qtype == QT_Q8_0 ? 1.08 : 1.0;
+  return 4.0 + (double)rounds * a.L.K * qf * (rt == 4 ? 2.5e-3 : rt == 2 ? 1.6e-3 : 0.8e-3);
 }
 
 size_t skinny_swiglu_workspace_bytes(int M, int N, int K) {

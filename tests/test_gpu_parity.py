@@ -227,6 +227,30 @@ def test_grouped_equals_separate_calls(cuda, M):
         assert orc.rel_err(y.cpu().numpy(), ref) <= TOL
 
 
+@pytest.mark.parametrize("M,K", [(5, 1024), (16, 4352), (32, 256), (33, 2304), (64, 1024), (65, 2048), (100, 1024)])
+def test_grouped_skinny_launches(cuda, M, K):
+    """Grouped calls on the skinny kernel (same-type weights side by side in one launch, at most
+    four) equal the skinny kernel's single calls bit for bit: ragged and single-row weights,
+    weights that end inside a slab, a bias, a second type, a fifth weight.  Above M = 32 the
+    estimates choose the kernel: narrow weights take the skinny one."""
+    import torch
+    specs = [(Q4K, 512), (Q4K, 130), (Q6K, 128), (Q4K, 1), (Q6K, 33), (Q4K, 640), (Q4K, 63)]
+    ws = [mx.pack_weights(mx.synth_gguf(qt, N, K, 500 + i), N, K, qt, device=cuda) for i, (qt, N) in enumerate(specs)]
+    x, _ = _act(torch, M, K, mx.BF16, 510, cuda)
+    bias = torch.linspace(-1, 1, 130, device=cuda).to(torch.bfloat16)
+    biases = [None, bias] + [None] * 5
+    ys = mx.q_gemm_dequant_grouped(x, ws, biases=biases, out_dtype=torch.float32)
+    try:
+        mx.qgemm.test_force_skinny(True)
+        y1 = [mx.q_gemm_dequant(x, w, M, w.N, K, w.qtype, bias=b, out_dtype=torch.float32, path=mx.PATH_MFMA)
+              for w, b in zip(ws, biases)]
+    finally:
+        mx.qgemm.test_force_skinny(False)
+    torch.cuda.synchronize()
+    for i in range(len(specs)):
+        assert torch.equal(ys[i], y1[i]), i
+
+
 @pytest.mark.parametrize("M,K", [(65, 1024), (130, 4096), (300, 2048), (48, 4096)])
 def test_grouped_tiled_launches(cuda, M, K):
     """Grouped calls on the tiled MFMA GEMM: same-type weights share one launch (tile columns
