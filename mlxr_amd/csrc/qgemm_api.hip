@@ -44,13 +44,15 @@ constexpr int kSkinnyOnlyMaxM = 32;
 int skinny_only_max_m() { return kSkinnyOnlyMaxM; }
 // Up to this M a call chooses between the skinny kernel (in blocks of 32 rows) and the tiled
 // one by their estimated times: on MI355X the skinny one is ahead for narrow weights, e.g.
-// Llama-3-8B k/v at M = 256 9.2 against 17.5 us.
-constexpr int kSkinnyMaxM = 256;
+// Llama-3-8B k/v at M = 256 9.2 against 17.5 us, at M = 512 13.9 against 22.1 us.
+constexpr int kSkinnyMaxM = 2048;
 
-// For skinny_only_max_m() < M <= kSkinnyMaxM: the kernel whose workspace size is reported, the
+// For skinny_only_max_m() < M <= kSizedMaxM: the kernel whose workspace size is reported, the
 // skinny one (true) or the tiled one.  Callers size their buffers by it, and
 // mlxr_qgemm_run_noalloc takes or refuses a call by them.
+constexpr int kSizedMaxM = 256;
 bool mid_sized_skinny(int M, const mlxr::PackedLayout& L) {
+  if (M > kSizedMaxM) return false;
   return mlxr::skinny_mb_est_us(M, L.N, L.K) < mlxr::mfma_est_us(M, L.N, L.K, L.qtype, ~(size_t)0);
 }
 void mid_workspace(int M, const mlxr::PackedLayout& L, size_t* bytes) {
@@ -239,7 +241,7 @@ int mlxr_qgemm_workspace_size(int qtype, int N, int K, int M, size_t* bytes) {
   if (rc) return rc;
   if (!bytes) return fail(MLXR_E_INVALID, "null output pointer");
   if (M < 0) return fail(MLXR_E_INVALID, "Input shape must be [M, K] (M=%d)", M);
-  if (M > skinny_only_max_m() && M <= kSkinnyMaxM)
+  if (M > skinny_only_max_m() && M <= kSizedMaxM)
     mid_workspace(M, L, bytes);
   else
     *bytes = M > skinny_only_max_m() ? mlxr::mfma_workspace_bytes(M, N, K)
@@ -295,7 +297,7 @@ int mlxr_qgemm_run_ws(int qtype, int N, int K, int group_size, const void* packe
   a.ws = workspace_dev;
   a.ws_bytes = workspace_dev ? workspace_bytes : 0;
   // GEMV (no MFMA) for decode (gemv_auto); MFMA kernels otherwise: the skinny one up to
-  // M = 32, then up to M = 256 the skinny or the tiled one, the tiled one above
+  // M = 32, then up to M = 2048 the skinny or the tiled one, the tiled one above
   // (MLXR_PATH_GEMV / MLXR_PATH_MFMA force the family)
   const bool gemv = path == MLXR_PATH_GEMV || (path == MLXR_PATH_AUTO && gemv_auto(M, a.L));
   // the skinny kernels address operands with 32-bit offsets; the tiled launcher splits
@@ -311,7 +313,7 @@ int mlxr_qgemm_run_ws(int qtype, int N, int K, int group_size, const void* packe
     size_t need = 0;
     mid_workspace(M, a.L, &need);
     const bool ws_ok = need == 0 || (a.ws && a.ws_bytes >= need);
-    if (!ws_ok) {
+    if (!ws_ok && M <= kSizedMaxM) {
       a.ws = nullptr;
       a.ws_bytes = 0;
     }
@@ -501,8 +503,9 @@ int mlxr_qgemm_grouped_workspace_size(int count, const mlxr_qgemm_item* items, i
 }  // extern "C"
 
 namespace {
-// How mlxr_qgemm_swiglu runs a shape: 0 GEMV launch (M <= 4), 1 narrow skinny kernel
-// (M <= 32), 2 tiled kernel, 3 unfused (operands of 2 GiB or more: two projections, then
+// How mlxr_qgemm_swiglu runs a shape: 0 GEMV launch (M <= 4), 1 skinny kernel
+// (M <= 32), 2 tiled kernel (or the skinny one, by the estimates: the workspace reported is the
+// tiled kernel's), 3 unfused (operands of 2 GiB or more: two projections, then
 // mlxr_swiglu with up in the workspace).  Kinds 1 and 2 fuse the gating into the
 // projection launch; their workspace only holds split-K partials.
 int swiglu_kind(const mlxr::RunArgs& a) {
@@ -556,7 +559,14 @@ int mlxr_qgemm_swiglu(int qtype, int N, int K, const void* gate_packed, const vo
   u.y = nullptr;
   g.y_dtype = u.y_dtype = h_dtype;
   g.M = u.M = M;
-  const int kind = swiglu_kind(g);
+  int kind = swiglu_kind(g);
+  if (kind == 2 && M <= kSkinnyMaxM && mlxr::skinny_fits(g)) {
+    // above M = 32 by the estimates of a weight with both projections' rows (5632 x 2048 Q4_K at
+    // M = 64, us, tiled / skinny: 19.9 / 16.2)
+    const mlxr::RunArgs* both[2] = {&g, &u};
+    const size_t have = workspace_dev && workspace_bytes >= need ? ~(size_t)0 : 0;
+    if (N <= INT32_MAX / 2 && mlxr::skinny_est_us(both, 2) < mlxr::mfma_est_us(M, 2 * N, K, qtype, have)) kind = 1;
+  }
   hipStream_t s = (hipStream_t)stream;
   if (kind == 0) {
     const hipError_t e = mlxr::launch_gemv_swiglu(g, u, s);

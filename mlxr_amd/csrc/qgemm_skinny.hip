@@ -658,7 +658,8 @@ double skinny_est_us(const RunArgs* const* items, int n) {
   const int cus = device_cu_count();
   const long rounds = (items_of(N, n, a.M, false, rt) + cus - 1) / cus;
   const double qf = a.L.qtype == QT_Q6_K ? 1.3 : a.L.qtype == QT_Q5_K ? 1.16 : a.L.qtype == QT_Q8_0 ? 1.08 : 1.0;
-  return 4.0 + (double)rounds * a.L.K * qf * (rt == 4 ? 2.5e-3 : rt == 2 ? 1.6e-3 : 0.8e-3);
+  const int k = (a.L.K + 2047) / 2048 * 2048;  // the 8 wavefronts' super-blocks: a rest takes as long
+  return 4.0 + (double)rounds * k * qf * (rt == 4 ? 2.5e-3 : rt == 2 ? 1.6e-3 : 0.8e-3);
 }
 
 size_t skinny_swiglu_workspace_bytes(int M, int N, int K) {

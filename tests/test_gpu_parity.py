@@ -251,6 +251,28 @@ def test_grouped_skinny_launches(cuda, M, K):
         assert torch.equal(ys[i], y1[i]), i
 
 
+@pytest.mark.parametrize("qt,M,N,K", [(Q4K, 33, 63, 256), (Q6K, 64, 130, 2304), (Q80, 100, 65, 1024), (Q40, 257, 48, 2048)])
+def test_swiglu_of_narrow_weights_takes_skinny_kernel(cuda, qt, M, N, K):
+    """Above M = 32 the fused SwiGLU of narrow weights runs on the skinny kernel: its sums are
+    those of the projections on that kernel, gated in fp32 (exp of g within 2 |g| + 8 units of
+    2^-23, a few more for the division and the products)."""
+    import torch
+    wg, pg = _packed(torch, qt, N, K, 611, cuda)
+    wu, pu = _packed(torch, qt, N, K, 612, cuda)
+    x, _ = _act(torch, M, K, mx.BF16, 613 + M, cuda)
+    h = mx.q_gemm_swiglu(x, pg, pu, out_dtype=torch.float32)
+    try:
+        mx.qgemm.test_force_skinny(True)
+        g, u = (mx.q_gemm_dequant(x, p, M, N, K, qt, out_dtype=torch.float32, path=mx.PATH_MFMA).double()
+                for p in (pg, pu))
+    finally:
+        mx.qgemm.test_force_skinny(False)
+    ref = g / (1 + torch.exp(-g)) * u
+    # gate values whose exp leaves the fp32 range give results below its normal numbers
+    bound = (16 + 2 * g.abs()) * 2.0**-23 * ref.abs() + 2.0**-126 * (1 + u.abs())
+    assert ((h.double() - ref).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("M,K", [(65, 1024), (130, 4096), (300, 2048), (48, 4096)])
 def test_grouped_tiled_launches(cuda, M, K):
     """Grouped calls on the tiled MFMA GEMM: same-type weights share one launch (tile columns
