@@ -66,7 +66,7 @@ enum {
                          (mlxr_qgemm_auto_path), M <= 4; MFMA kernels above: skinny
                          (weights streamed once) for M <= 64, tiled GEMM beyond.  When
                          mlxr_qgemm_run_ws is given the workspace it asks for, calls with
-                         32 < M <= 256 take whichever of the two is estimated faster for
+                         32 < M <= 2048 take whichever of the two is estimated faster for
                          the shape (the skinny one for narrow weights) */
   MLXR_PATH_GEMV = 1, /* force the wavefront-reduction GEMV kernel (any M <= 64) */
   MLXR_PATH_MFMA = 2  /* force the MFMA kernels (chosen as for MLXR_PATH_AUTO) */
@@ -127,12 +127,13 @@ int mlxr_qgemm_run_ex(int qtype, int N, int K, int group_size, const void* packe
                       void* y_dev, int y_dtype, int M, int path, void* stream);
 
 /* Device workspace bytes mlxr_qgemm_run_ws can use for an [M, N, K] problem; 0 when the
- * problem would not use one.  MFMA GEMMs whose workgroups would be too few to fill the
- * device (tiled ones, M > 32, and skinny ones with few 32-row slabs) split K over several
- * workgroups and add the fp32 partials in a second kernel; the workspace holds those
- * partials (splits x M x N x 4 bytes).  For 32 < M <= 256 the size is that of the kernel
- * the call would choose with it; mlxr_qgemm_run_ws ignores a smaller workspace (the call
- * then runs as mlxr_qgemm_run_ex: skinny kernel for M <= 64, tiled one above, unsplit).
+ * problem would not use one.  Tiled MFMA GEMMs (M > 32) whose workgroups would be too few to
+ * fill the device split K over several workgroups and add the fp32 partials in a second
+ * kernel; the workspace holds those partials (splits x M x N x 4 bytes).  The skinny kernel
+ * leaves it untouched (a size is reported for some of its shapes too).  With the reported size,
+ * calls with 32 < M <= 2048 run the skinny or the tiled kernel, whichever is estimated faster;
+ * up to M = 256 mlxr_qgemm_run_ws ignores a smaller workspace (the call then runs as
+ * mlxr_qgemm_run_ex: skinny kernel for M <= 64, tiled one above, unsplit).
  * When the size is 0 the call makes the same choice with or without a workspace.
  * No counterpart in the reference (its kernel has no K split, q_gemm_dequant.metal:374-464). */
 int mlxr_qgemm_workspace_size(int qtype, int N, int K, int M, size_t* bytes);
@@ -196,7 +197,7 @@ typedef struct mlxr_qgemm_item {
 int mlxr_qgemm_run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,
                            void* stream);
 /* mlxr_qgemm_run_grouped with a caller-owned device workspace (NULL or too small = as
- * mlxr_qgemm_run_grouped).  With it, launches at 32 < M <= 256 go to the skinny or the
+ * mlxr_qgemm_run_grouped).  With it, launches at 32 < M <= 2048 go to the skinny or the
  * tiled kernel, whichever is estimated faster for the weights together, the tiled launches split
  * K over the concatenated N of their weights when their tiles cannot fill the device, and single
  * items run as mlxr_qgemm_run_ws.  Results then differ from separate calls only in
