@@ -271,10 +271,20 @@ int mlxr_qgemm_mlp_status(void* workspace_dev, void* stream);
  * by tests to exercise the timeout path.  mlxr_qgemm_test_force_skinny(1): every call of the
  * MFMA family (M > 4, or MLXR_PATH_MFMA) runs the skinny kernel, at any M, until called
  * with 0; tests use it to reach the skinny kernel's blocks of M at shapes the automatic
- * choice gives to the tiled kernel.  mlxr_qgemm_test_skinny_stage: weight tiles a wavefront of
+ * choice gives to the tiled kernel; mlxr_qgemm_test_force_tiled(1) likewise sends them to the
+ * tiled kernel (split over K where the call's workspace holds its partials).
+ * mlxr_qgemm_test_skinny_stage: weight tiles a wavefront of
  * the skinny kernel takes: 0 one, 2 two, 3 and above four (SwiGLU: two, two, four), 1 restores
  * the choice by shape; tests use it to check every variant against the oracle.
- * All are process-wide (atomics). */
+ * All are process-wide (atomics).
+ * mlxr_qgemm_test_kernels launches nothing: it tells which kernel would run each item, and which
+ * items share a launch (equal numbers in launches), of call 0 mlxr_qgemm_run_ws for each item,
+ * 1 mlxr_qgemm_run_grouped_ws, 2 mlxr_qgemm_swiglu with items[0] as gate and up (count 1), given a
+ * workspace of workspace_bytes (0: none).  Only the items' qtype, N and K are read. */
+enum { MLXR_KERNEL_GEMV = 0, MLXR_KERNEL_SKINNY = 1, MLXR_KERNEL_TILED = 2, MLXR_KERNEL_TILED_SPLIT = 3 };
+int mlxr_qgemm_test_kernels(int call, int count, const mlxr_qgemm_item* items, int M, size_t workspace_bytes,
+                            int* kernels, int* launches);
+int mlxr_qgemm_test_force_tiled(int on);
 int mlxr_qgemm_test_set_operand_limit(size_t bytes);
 int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks);
 int mlxr_qgemm_test_force_skinny(int on);

@@ -41,13 +41,12 @@ bool gemv_auto(int M, const mlxr::PackedLayout& L) {
 // 10.6, 4096 x 4096 10.2 / 15.0, 4096 x 14336 24.1 / 24.9, 14336 x 4096 25.9 / 24.1; at M = 24
 // the last takes it 15.7).
 constexpr int kSkinnyOnlyMaxM = 32;
-int skinny_only_max_m() { return kSkinnyOnlyMaxM; }
 // Up to this M a call chooses between the skinny kernel (in blocks of 32 rows) and the tiled
 // one by their estimated times: on MI355X the skinny one is ahead for narrow weights, e.g.
 // Llama-3-8B k/v at M = 256 9.2 against 17.5 us, at M = 512 13.9 against 22.1 us.
 constexpr int kSkinnyMaxM = 2048;
 
-// For skinny_only_max_m() < M <= kSizedMaxM: the kernel whose workspace size is reported, the
+// For kSkinnyOnlyMaxM < M <= kSizedMaxM: the kernel whose workspace size is reported, the
 // skinny one (true) or the tiled one.  Callers size their buffers by it, and
 // mlxr_qgemm_run_noalloc takes or refuses a call by them.
 constexpr int kSizedMaxM = 256;
@@ -55,11 +54,49 @@ bool mid_sized_skinny(int M, const mlxr::PackedLayout& L) {
   if (M > kSizedMaxM) return false;
   return mlxr::skinny_mb_est_us(M, L.N, L.K) < mlxr::mfma_est_us(M, L.N, L.K, L.qtype, ~(size_t)0);
 }
-void mid_workspace(int M, const mlxr::PackedLayout& L, size_t* bytes) {
-  *bytes = mid_sized_skinny(M, L) ? mlxr::skinny_workspace_bytes(M, L.N, L.K, L.qtype)
-                                  : mlxr::mfma_workspace_bytes(M, L.N, L.K);
+size_t single_workspace(int M, const mlxr::PackedLayout& L) {
+  const bool skinny = M <= kSkinnyOnlyMaxM ? !gemv_auto(M, L) : mid_sized_skinny(M, L);
+  if (skinny) return mlxr::skinny_workspace_bytes(M, L.N, L.K, L.qtype);
+  return M <= kSkinnyOnlyMaxM ? 0 : mlxr::mfma_workspace_bytes(M, L.N, L.K);
 }
-std::atomic<int> g_force_skinny{0};
+// The kernel tests force on calls of the MFMA family.
+enum Forced { kNotForced, kForceSkinny, kForceTiled };
+std::atomic<int> g_forced{kNotForced};
+int forced() { return g_forced.load(std::memory_order_relaxed); }
+
+// The kernel of a single call: GEMV (no MFMA) for decode (gemv_auto); MFMA kernels otherwise, the
+// skinny one up to M = 32, then up to M = 2048 the skinny or the tiled one, the tiled one above
+// (MLXR_PATH_GEMV / MLXR_PATH_MFMA force the family).  The skinny kernel addresses operands with
+// 32-bit offsets; the tiled launcher splits larger problems into chunks.  Clears a.ws where the
+// call does not use its workspace.
+enum Kernel { kGemv, kSkinny, kTiled };
+Kernel single_kernel(mlxr::RunArgs& a, int path) {
+  const int M = a.M;
+  if (path == MLXR_PATH_GEMV || (path == MLXR_PATH_AUTO && gemv_auto(M, a.L))) return kGemv;
+  const bool fits = mlxr::skinny_fits(a);
+  if (forced() != kNotForced) return forced() == kForceSkinny && fits ? kSkinny : kTiled;
+  if (M <= kSkinnyOnlyMaxM) return fits ? kSkinny : kTiled;
+  if (M > kSkinnyMaxM) return kTiled;
+  // a workspace below the size mlxr_qgemm_workspace_size asks for is not used; a call
+  // whose size is 0 has what it asks for, with or without one
+  const size_t need = single_workspace(M, a.L);
+  const bool ws_ok = need == 0 || (a.ws && a.ws_bytes >= need);
+  if (!ws_ok && M <= kSizedMaxM) {
+    a.ws = nullptr;
+    a.ws_bytes = 0;
+  }
+  if (!fits) return kTiled;
+  // with it, the tiled kernel runs where its size was reported and it is estimated to be
+  // ahead (4096 x 4096 Q4_K, us, tiled / skinny: M = 64 18.1 / 10.7, M = 128 23.7 / 14.4, M =
+  // 256 26.9 / 24.6; 14336 x 4096: M = 64 25.9 / 26.2, M = 128 33.4 / 47.6); without, the
+  // skinny one takes M <= 64 and the tiled one (unsplit) larger M
+  if (!ws_ok) return M <= 64 ? kSkinny : kTiled;
+  const mlxr::RunArgs* one[1] = {&a};
+  return mid_sized_skinny(M, a.L) ||
+                 mlxr::skinny_est_us(one, 1) < mlxr::mfma_est_us(M, a.L.N, a.L.K, a.L.qtype, ~(size_t)0)
+             ? kSkinny
+             : kTiled;
+}
 
 thread_local std::string g_err;
 
@@ -241,12 +278,7 @@ int mlxr_qgemm_workspace_size(int qtype, int N, int K, int M, size_t* bytes) {
   if (rc) return rc;
   if (!bytes) return fail(MLXR_E_INVALID, "null output pointer");
   if (M < 0) return fail(MLXR_E_INVALID, "Input shape must be [M, K] (M=%d)", M);
-  if (M > skinny_only_max_m() && M <= kSizedMaxM)
-    mid_workspace(M, L, bytes);
-  else
-    *bytes = M > skinny_only_max_m() ? mlxr::mfma_workspace_bytes(M, N, K)
-             : !gemv_auto(M, L)      ? mlxr::skinny_workspace_bytes(M, N, K, qtype)
-                                     : 0;
+  *bytes = single_workspace(M, L);
   return MLXR_OK;
 }
 
@@ -296,41 +328,12 @@ int mlxr_qgemm_run_ws(int qtype, int N, int K, int group_size, const void* packe
   a.M = M;
   a.ws = workspace_dev;
   a.ws_bytes = workspace_dev ? workspace_bytes : 0;
-  // GEMV (no MFMA) for decode (gemv_auto); MFMA kernels otherwise: the skinny one up to
-  // M = 32, then up to M = 2048 the skinny or the tiled one, the tiled one above
-  // (MLXR_PATH_GEMV / MLXR_PATH_MFMA force the family)
-  const bool gemv = path == MLXR_PATH_GEMV || (path == MLXR_PATH_AUTO && gemv_auto(M, a.L));
-  // the skinny kernels address operands with 32-bit offsets; the tiled launcher splits
-  // larger problems into chunks
-  bool skinny = false;
-  if (!gemv && g_force_skinny.load(std::memory_order_relaxed)) {
-    skinny = mlxr::skinny_fits(a);
-  } else if (!gemv && M <= skinny_only_max_m()) {
-    skinny = mlxr::skinny_fits(a);
-  } else if (!gemv && M <= kSkinnyMaxM) {
-    // a workspace below the size mlxr_qgemm_workspace_size asks for is not used; a call
-    // whose size is 0 has what it asks for, with or without one
-    size_t need = 0;
-    mid_workspace(M, a.L, &need);
-    const bool ws_ok = need == 0 || (a.ws && a.ws_bytes >= need);
-    if (!ws_ok && M <= kSizedMaxM) {
-      a.ws = nullptr;
-      a.ws_bytes = 0;
-    }
-    // with it, the tiled kernel runs where its size was reported and it is estimated to be
-    // ahead (4096 x 4096 Q4_K, us, tiled / skinny: M = 64 18.1 / 10.7, M = 128 23.7 / 14.4, M =
-    // 256 26.9 / 24.6; 14336 x 4096: M = 64 25.9 / 26.2, M = 128 33.4 / 47.6); without, the
-    // skinny one takes M <= 64 and the tiled one (unsplit) larger M
-    const mlxr::RunArgs* one[1] = {&a};
-    skinny = mlxr::skinny_fits(a) &&
-             (ws_ok ? mid_sized_skinny(M, a.L) || mlxr::skinny_est_us(one, 1) < mlxr::mfma_est_us(M, N, K, qtype, ~(size_t)0)
-                    : M <= 64);
-  }
+  const Kernel k = single_kernel(a, path);
   hipError_t e;
-  if (gemv) e = mlxr::launch_gemv(a, (hipStream_t)stream);
-  else if (skinny) e = mlxr::launch_skinny(a, (hipStream_t)stream);
+  if (k == kGemv) e = mlxr::launch_gemv(a, (hipStream_t)stream);
+  else if (k == kSkinny) e = mlxr::launch_skinny(a, (hipStream_t)stream);
   else e = mlxr::launch_mfma(a, (hipStream_t)stream);
-  if (e != hipSuccess) return hip_fail(e, gemv ? "gemv launch" : "mfma launch");
+  if (e != hipSuccess) return hip_fail(e, k == kGemv ? "gemv launch" : "mfma launch");
   return MLXR_OK;
 }
 
@@ -356,15 +359,17 @@ struct Batch {
   int idx[4];
   int n;
 };
-// The batches a workspace is sized for: those of `sized`, where only GEMV and tiled launches
-// (with_ws, or M > 64) take several items.
+// `sized`: the batches the reported workspace is sized for, where only GEMV and tiled launches take
+// several items.  Otherwise those a call runs: with a workspace, every item the tiled kernel
+// can take at M > 32 joins a tiled batch (whose kernel batch_skinny picks).
 std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool with_ws, bool sized) {
   const int count = (int)a.size();
-  const bool tiled = M > 64 || (M > skinny_only_max_m() && with_ws);
   auto kind_of = [&](const mlxr::RunArgs& r) {
     if (M <= kGemvMaxM && grouped_gemv(M, r)) return kGroupedGemv;
-    if (tiled) return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
-    return !sized && !gemv_auto(M, r.L) && mlxr::skinny_fits(r) ? kGroupedSkinny : kSingle;
+    if (M > kSkinnyOnlyMaxM && (with_ws || sized)) return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
+    if (sized) return kSingle;
+    if (M > 64) return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
+    return !gemv_auto(M, r.L) && mlxr::skinny_fits(r) ? kGroupedSkinny : kSingle;
   };
   std::vector<bool> done((size_t)count, false);
   std::vector<Batch> out;
@@ -388,14 +393,47 @@ std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool
 // estimates of a single weight with the batch's columns (Llama-3-8B q,k,v Q4_K at M = 64, us,
 // tiled / skinny: 23.0 / 14.6).
 bool batch_skinny(const mlxr::RunArgs* const* items, int n, int M, size_t ws_bytes) {
-  if (M > kSkinnyMaxM) return false;
+  if (forced() == kForceTiled) return false;
+  if (M > kSkinnyMaxM && forced() != kForceSkinny) return false;
   int cols = 0;
   for (int i = 0; i < n; ++i) {
     if (!mlxr::skinny_fits(*items[i])) return false;
     if (items[i]->L.N > INT32_MAX / 4) return false;
     cols += items[i]->L.N;
   }
+  if (forced() == kForceSkinny) return true;
   return mlxr::skinny_est_us(items, n) < mlxr::mfma_est_us(M, cols, items[0]->L.K, items[0]->L.qtype, ws_bytes);
+}
+
+// The workspace reported for a grouped call.
+size_t grouped_need(const std::vector<mlxr::RunArgs>& a, int M) {
+  size_t need = 0;
+  for (const Batch& bt : plan_batches(a, M, true, true)) {
+    const mlxr::RunArgs* batch[4];
+    for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
+    size_t b = 0;
+    if (bt.kind == kGroupedTiled) b = mlxr::mfma_grouped_workspace_bytes(batch, bt.n);
+    else if (bt.kind == kSingle) b = single_workspace(M, batch[0]->L);
+    need = std::max(need, b);
+  }
+  return need;
+}
+
+// The batches of a call and their kernels (kGroupedTiled / kGroupedSkinny decided).  A workspace
+// below the reported size is none, and so is one of a call whose size is 0: *ws is cleared.
+std::vector<Batch> call_batches(const std::vector<mlxr::RunArgs>& a, int M, void** ws, size_t ws_bytes) {
+  if (*ws) {
+    const size_t need = grouped_need(a, M);
+    if (need == 0 || ws_bytes < need) *ws = nullptr;
+  }
+  std::vector<Batch> out = plan_batches(a, M, *ws != nullptr, false);
+  for (Batch& bt : out) {
+    if (bt.kind != kGroupedTiled || !*ws) continue;
+    const mlxr::RunArgs* batch[4];
+    for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
+    if (batch_skinny(batch, bt.n, M, ws_bytes)) bt.kind = kGroupedSkinny;
+  }
+  return out;
 }
 
 // Validates the items (each exactly as a single call) and fills their run arguments.
@@ -439,13 +477,13 @@ int run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int 
   int rc = grouped_args(count, items, x_dev, x_dtype, M, true, stream, a);
   if (rc || count == 0 || M == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
-  for (const Batch& bt : plan_batches(a, M, ws != nullptr, false)) {
+  for (const Batch& bt : call_batches(a, M, &ws, ws_bytes)) {
     const mlxr::RunArgs* batch[4];
     for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
     if (bt.kind == kGroupedGemv) {
       const hipError_t e = mlxr::launch_gemv_grouped(batch, bt.n, s);
       if (e != hipSuccess) return hip_fail(e, "grouped gemv launch");
-    } else if (bt.kind == kGroupedSkinny || (bt.kind == kGroupedTiled && ws && batch_skinny(batch, bt.n, M, ws_bytes))) {
+    } else if (bt.kind == kGroupedSkinny) {
       const hipError_t e = mlxr::launch_skinny_grouped(batch, bt.n, s);
       if (e != hipSuccess) return hip_fail(e, "grouped skinny launch");
     } else if (bt.kind == kGroupedTiled) {
@@ -480,23 +518,7 @@ int mlxr_qgemm_grouped_workspace_size(int count, const mlxr_qgemm_item* items, i
   std::vector<mlxr::RunArgs> a;
   int rc = grouped_args(count, items, nullptr, MLXR_BF16, M, false, nullptr, a);
   if (rc) return rc;
-  size_t need = 0;
-  if (count > 0 && M > 0) {
-    for (const Batch& bt : plan_batches(a, M, true, true)) {
-      const mlxr::RunArgs* batch[4];
-      for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
-      size_t b = 0;
-      if (bt.kind == kGroupedTiled) {
-        b = mlxr::mfma_grouped_workspace_bytes(batch, bt.n);
-      } else if (bt.kind == kSingle) {
-        const mlxr_qgemm_item& it = items[bt.idx[0]];
-        rc = mlxr_qgemm_workspace_size(it.qtype, it.N, it.K, M, &b);
-        if (rc) return rc;
-      }
-      need = std::max(need, b);
-    }
-  }
-  *bytes = need;
+  *bytes = count > 0 && M > 0 ? grouped_need(a, M) : 0;
   return MLXR_OK;
 }
 
@@ -512,6 +534,18 @@ int swiglu_kind(const mlxr::RunArgs& a) {
   if (a.M <= kGemvMaxM && gemv_auto(a.M, a.L) && mlxr::gemv_groupable(a)) return 0;
   if (!mlxr::mfma_groupable(a)) return 3;
   return a.M <= kSkinnyOnlyMaxM ? 1 : 2;
+}
+// The kind a call runs as: above M = 32 by the estimates of a weight with both projections' rows
+// (5632 x 2048 Q4_K at M = 64, us, tiled / skinny: 19.9 / 16.2).  ws: the call has the workspace
+// that its size asks for.
+int swiglu_kernel(const mlxr::RunArgs& g, const mlxr::RunArgs& u, bool ws) {
+  const int kind = swiglu_kind(g), M = g.M, N = g.L.N, K = g.L.K;
+  if (kind == 0 || kind == 3) return kind;
+  if (forced() != kNotForced) return forced() == kForceTiled ? 2 : mlxr::skinny_fits(g) ? 1 : 2;
+  if (kind == 1 || M > kSkinnyMaxM || !mlxr::skinny_fits(g) || N > INT32_MAX / 2) return kind;
+  const mlxr::RunArgs* both[2] = {&g, &u};
+  const size_t have = ws ? ~(size_t)0 : 0;
+  return mlxr::skinny_est_us(both, 2) < mlxr::mfma_est_us(M, 2 * N, K, g.L.qtype, have) ? 1 : 2;
 }
 }  // namespace
 
@@ -559,14 +593,7 @@ int mlxr_qgemm_swiglu(int qtype, int N, int K, const void* gate_packed, const vo
   u.y = nullptr;
   g.y_dtype = u.y_dtype = h_dtype;
   g.M = u.M = M;
-  int kind = swiglu_kind(g);
-  if (kind == 2 && M <= kSkinnyMaxM && mlxr::skinny_fits(g)) {
-    // above M = 32 by the estimates of a weight with both projections' rows (5632 x 2048 Q4_K at
-    // M = 64, us, tiled / skinny: 19.9 / 16.2)
-    const mlxr::RunArgs* both[2] = {&g, &u};
-    const size_t have = workspace_dev && workspace_bytes >= need ? ~(size_t)0 : 0;
-    if (N <= INT32_MAX / 2 && mlxr::skinny_est_us(both, 2) < mlxr::mfma_est_us(M, 2 * N, K, qtype, have)) kind = 1;
-  }
+  const int kind = swiglu_kernel(g, u, workspace_dev && workspace_bytes >= need);
   hipStream_t s = (hipStream_t)stream;
   if (kind == 0) {
     const hipError_t e = mlxr::launch_gemv_swiglu(g, u, s);
@@ -746,7 +773,68 @@ int mlxr_qgemm_test_skinny_stage(int on) {
 }
 
 int mlxr_qgemm_test_force_skinny(int on) {
-  g_force_skinny.store(on ? 1 : 0, std::memory_order_relaxed);
+  g_forced.store(on ? kForceSkinny : kNotForced, std::memory_order_relaxed);
+  return MLXR_OK;
+}
+
+int mlxr_qgemm_test_force_tiled(int on) {
+  g_forced.store(on ? kForceTiled : kNotForced, std::memory_order_relaxed);
+  return MLXR_OK;
+}
+
+int mlxr_qgemm_test_kernels(int call, int count, const mlxr_qgemm_item* items, int M, size_t workspace_bytes,
+                            int* kernels, int* launches) {
+  if (call < 0 || call > 2 || (call == 2 && count != 1) || !kernels || !launches || M < 1)
+    return fail(MLXR_E_INVALID, "invalid kernel query");
+  std::vector<mlxr::RunArgs> a;
+  const int rc = grouped_args(count, items, nullptr, MLXR_BF16, M, false, nullptr, a);
+  if (rc) return rc;
+  void* const ws = workspace_bytes ? (void*)items : nullptr;  // only compared with null
+  auto single = [&](int i) {
+    mlxr::RunArgs one = a[(size_t)i];
+    one.ws = ws;
+    one.ws_bytes = workspace_bytes;
+    const Kernel k = single_kernel(one, MLXR_PATH_AUTO);
+    if (k != kTiled) return k == kGemv ? MLXR_KERNEL_GEMV : MLXR_KERNEL_SKINNY;
+    const size_t need = mlxr::mfma_groupable(one) ? mlxr::mfma_workspace_bytes(M, one.L.N, one.L.K) : 0;
+    return need && one.ws && one.ws_bytes >= need ? MLXR_KERNEL_TILED_SPLIT : MLXR_KERNEL_TILED;
+  };
+  if (call == 0) {
+    for (int i = 0; i < count; ++i) {
+      kernels[i] = single(i);
+      launches[i] = i;
+    }
+  } else if (call == 1) {
+    void* gws = ws;
+    int launch = 0;
+    for (const Batch& bt : call_batches(a, M, &gws, workspace_bytes)) {
+      const mlxr::RunArgs* batch[4];
+      for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
+      const bool split = bt.kind == kGroupedTiled && gws && mlxr::mfma_grouped_workspace_bytes(batch, bt.n) > 0;
+      for (int k = 0; k < bt.n; ++k) {
+        const int i = bt.idx[k];
+        kernels[i] = bt.kind == kGroupedGemv     ? MLXR_KERNEL_GEMV
+                     : bt.kind == kGroupedSkinny ? MLXR_KERNEL_SKINNY
+                     : bt.kind == kSingle        ? single(i)
+                     : split                     ? MLXR_KERNEL_TILED_SPLIT
+                                                 : MLXR_KERNEL_TILED;
+        launches[i] = launch;
+      }
+      ++launch;
+    }
+  } else {
+    const mlxr_qgemm_item& it = items[0];
+    size_t need = 0;
+    mlxr_qgemm_swiglu_workspace_size(it.qtype, it.N, it.K, M, MLXR_BF16, &need);
+    const bool have = workspace_bytes && workspace_bytes >= need;
+    const int kind = swiglu_kernel(a[0], a[0], have);
+    kernels[0] = kind == 0   ? MLXR_KERNEL_GEMV
+                 : kind == 1 ? MLXR_KERNEL_SKINNY
+                 : kind == 2 && have && mlxr::mfma_swiglu_workspace_bytes(M, it.N, it.K) > 0
+                     ? MLXR_KERNEL_TILED_SPLIT
+                     : MLXR_KERNEL_TILED;
+    launches[0] = 0;
+  }
   return MLXR_OK;
 }
 

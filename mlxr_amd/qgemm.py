@@ -87,6 +87,8 @@ _SIGS = {
     "mlxr_qgemm_test_set_operand_limit": (ctypes.c_int, [ctypes.c_size_t]),
     "mlxr_qgemm_test_set_mlp_spin_limit": (ctypes.c_int, [ctypes.c_uint]),
     "mlxr_qgemm_test_force_skinny": (ctypes.c_int, [ctypes.c_int]),
+    "mlxr_qgemm_test_force_tiled": (ctypes.c_int, [ctypes.c_int]),
+    "mlxr_qgemm_test_kernels": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_void_p]),
     "mlxr_qgemm_test_skinny_stage": (ctypes.c_int, [ctypes.c_int]),
     "mlxr_qgemm_auto_path": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                              ctypes.POINTER(ctypes.c_int)]),
@@ -442,6 +444,26 @@ def test_force_skinny(on):
     """Test hook: send every MFMA-family call to the skinny kernel (any M, in blocks
     of M) while on."""
     _check(lib().mlxr_qgemm_test_force_skinny(1 if on else 0))
+
+
+def test_force_tiled(on):
+    """Test hook: send every MFMA-family call to the tiled kernel while on."""
+    _check(lib().mlxr_qgemm_test_force_tiled(1 if on else 0))
+
+
+KERNEL_GEMV, KERNEL_SKINNY, KERNEL_TILED, KERNEL_TILED_SPLIT = 0, 1, 2, 3
+
+
+def test_kernels(call, weights, M, workspace_bytes=0):
+    """Test hook: the kernel (KERNEL_*) of each (qtype, N, K) of `weights`, and the number of the launch
+    it is part of, for call "single", "grouped" or "swiglu" with a workspace of that size.
+    Launches nothing."""
+    n = len(weights)
+    arr = (Item * n)(*[Item(int(qt), N, K, 0, None, None, F32, None, F32) for qt, N, K in weights])
+    kernels, launches = (ctypes.c_int * n)(), (ctypes.c_int * n)()
+    _check(lib().mlxr_qgemm_test_kernels({"single": 0, "grouped": 1, "swiglu": 2}[call], n, arr, int(M),
+                                         int(workspace_bytes), kernels, launches))
+    return list(kernels), list(launches)
 
 
 def test_skinny_stage(mode):

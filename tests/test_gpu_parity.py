@@ -307,6 +307,40 @@ def test_grouped_tiled_launches(cuda, M, K):
         assert orc.rel_err(y.cpu().numpy(), ref) <= TOL, i
 
 
+@pytest.mark.parametrize("M,K", [(33, 2304), (100, 4096), (333, 2048)])
+def test_grouped_call_with_short_workspace(cuda, M, K):
+    """A grouped call whose workspace is one byte, or one byte below its size, equals
+    mlxr_qgemm_run_grouped bit for bit."""
+    import torch
+    Ns = [512, 130, 1024]
+    ws = [mx.pack_weights(mx.synth_gguf(Q4K, N, K, 700 + i), N, K, Q4K, device=cuda) for i, N in enumerate(Ns)]
+    x, _ = _act(torch, M, K, mx.BF16, 710, cuda)
+    L, s = mx.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def call(nbytes):
+        ys = [torch.full((M, N), float("nan"), device=cuda) for N in Ns]
+        arr = (mx.qgemm.Item * 3)(*[mx.qgemm.Item(int(Q4K), N, K, 0, w.data_ptr(), None, mx.F32, y.data_ptr(), mx.F32)
+                                    for N, w, y in zip(Ns, ws, ys)])
+        if nbytes is None:
+            rc = L.mlxr_qgemm_run_grouped(3, arr, x.data_ptr(), mx.BF16, M, s)
+        else:
+            if nbytes < 0:
+                need = ctypes.c_size_t(0)
+                assert L.mlxr_qgemm_grouped_workspace_size(3, arr, M, ctypes.byref(need)) == 0
+                assert need.value > 0
+                nbytes += need.value
+            buf = torch.empty(nbytes, dtype=torch.uint8, device=cuda)
+            rc = L.mlxr_qgemm_run_grouped_ws(3, arr, x.data_ptr(), mx.BF16, M, buf.data_ptr(), nbytes, s)
+        assert rc == 0, L.mlxr_qgemm_last_error()
+        torch.cuda.synchronize()
+        return ys
+
+    none = call(None)
+    for nbytes in (1, -1):
+        for y, y0 in zip(call(nbytes), none):
+            assert torch.equal(y, y0), nbytes
+
+
 @pytest.mark.parametrize("ydt", ["bf16", "f32"])
 def test_grouped_split_reduce_vectorized(cuda, ydt):
     """Grouped tiled launch split over K whose weights all have N % 4 == 0 (the reduce then
