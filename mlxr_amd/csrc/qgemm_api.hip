@@ -361,15 +361,22 @@ struct Batch {
 };
 // `sized`: the batches the reported workspace is sized for, where only GEMV and tiled launches take
 // several items.  Otherwise those a call runs: with a workspace, every item the tiled kernel
-// can take at M > 32 joins a tiled batch (whose kernel batch_skinny picks).
+// can take at M > 32 joins a tiled batch (whose kernel batch_skinny picks); without, items whose
+// single calls run on the same kernel share a launch, so their results are those calls'.
 std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool with_ws, bool sized) {
   const int count = (int)a.size();
   auto kind_of = [&](const mlxr::RunArgs& r) {
     if (M <= kGemvMaxM && grouped_gemv(M, r)) return kGroupedGemv;
     if (M > kSkinnyOnlyMaxM && (with_ws || sized)) return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
     if (sized) return kSingle;
-    if (M > 64) return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
-    return !gemv_auto(M, r.L) && mlxr::skinny_fits(r) ? kGroupedSkinny : kSingle;
+    mlxr::RunArgs one = r;
+    one.ws = nullptr;
+    one.ws_bytes = 0;
+    switch (single_kernel(one, MLXR_PATH_AUTO)) {
+      case kSkinny: return kGroupedSkinny;
+      case kTiled: return mlxr::mfma_groupable(r) ? kGroupedTiled : kSingle;
+      default: return kSingle;
+    }
   };
   std::vector<bool> done((size_t)count, false);
   std::vector<Batch> out;

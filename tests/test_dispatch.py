@@ -43,3 +43,16 @@ def test_grouped_workspace_below_its_size_is_none(g):
         none = qgemm.test_kernels("grouped", GROUPS[g], M)
         for nbytes in (1, need // 2, need - 1) if need else (1, 1 << 30):
             assert qgemm.test_kernels("grouped", GROUPS[g], M, nbytes) == none, (M, need, nbytes)
+
+
+@pytest.mark.parametrize("g", range(len(GROUPS)))
+def test_grouped_without_workspace_takes_kernels_of_single_calls(g):
+    """Without a workspace a grouped call equals separate calls bit for bit (M > 4): every item
+    runs on the kernel of its own call, and items of different types or kernels share no launch."""
+    for M in MS:
+        kernels, launches = qgemm.test_kernels("grouped", GROUPS[g], M)
+        assert kernels == qgemm.test_kernels("single", GROUPS[g], M)[0], M
+        for i in range(len(kernels)):
+            together = [j for j in range(len(kernels)) if launches[j] == launches[i]]
+            assert len(together) <= 4
+            assert {(kernels[j], GROUPS[g][j][0]) for j in together} == {(kernels[i], GROUPS[g][i][0])}, M

@@ -340,6 +340,24 @@ def test_grouped_call_with_short_workspace(cuda, M, K):
         for y, y0 in zip(call(nbytes), none):
             assert torch.equal(y, y0), nbytes
 
+@pytest.mark.parametrize("specs,M,K", [([(Q4K, 512), (Q4K, 33), (Q6K, 130)], 300, 256), ([(Q80, 65536), (Q80, 65)], 48, 2048),
+                                       ([(Q6K, 5632), (Q6K, 5632)], 512, 2048), ([(Q4K, 1024), (Q6K, 512)], 64, 4096)])
+def test_grouped_without_workspace_equals_single_calls(cuda, specs, M, K):
+    """mlxr_qgemm_run_grouped equals mlxr_qgemm_run for each weight bit for bit, also where a single
+    call's workspace size is 0 and the kernel is chosen by estimates."""
+    import torch
+    pws = [mx.pack_weights(mx.synth_gguf(qt, N, K, 720 + i), N, K, qt, device=cuda) for i, (qt, N) in enumerate(specs)]
+    x, _ = _act(torch, M, K, mx.BF16, 730, cuda)
+    ys = mx.q_gemm_dequant_grouped(x, pws, out_dtype=torch.float32, workspace=False)
+    L, s = mx.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for (qt, N), w, y in zip(specs, pws, ys):
+        y1 = torch.empty_like(y)
+        rc = L.mlxr_qgemm_run(int(qt), N, K, 0, w.data_ptr(), x.data_ptr(), mx.BF16, None, mx.F32, y1.data_ptr(),
+                              mx.F32, M, s)
+        assert rc == 0, L.mlxr_qgemm_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(y, y1), (str(qt), N)
+
 
 @pytest.mark.parametrize("ydt", ["bf16", "f32"])
 def test_grouped_split_reduce_vectorized(cuda, ydt):
