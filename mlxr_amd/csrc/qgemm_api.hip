@@ -385,8 +385,11 @@ std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool
     Batch bt{kind_of(a[i]), {i, 0, 0, 0}, 1};
     done[i] = true;
     if (bt.kind != kSingle) {
+      const mlxr::RunArgs* batch[4] = {&a[i]};
       for (int j = i + 1; j < count && bt.n < 4; ++j) {
         if (done[j] || a[j].L.qtype != a[i].L.qtype || kind_of(a[j]) != bt.kind) continue;
+        batch[bt.n] = &a[j];
+        if (bt.kind == kGroupedSkinny && !mlxr::skinny_group_fits(batch, bt.n + 1)) continue;
         bt.idx[bt.n++] = j;
         done[j] = true;
       }
@@ -402,9 +405,9 @@ std::vector<Batch> plan_batches(const std::vector<mlxr::RunArgs>& a, int M, bool
 bool batch_skinny(const mlxr::RunArgs* const* items, int n, int M, size_t ws_bytes) {
   if (forced() == kForceTiled) return false;
   if (M > kSkinnyMaxM && forced() != kForceSkinny) return false;
+  if (!mlxr::skinny_group_fits(items, n)) return false;
   int cols = 0;
   for (int i = 0; i < n; ++i) {
-    if (!mlxr::skinny_fits(*items[i])) return false;
     if (items[i]->L.N > INT32_MAX / 4) return false;
     cols += items[i]->L.N;
   }

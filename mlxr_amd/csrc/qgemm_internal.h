@@ -77,7 +77,7 @@ size_t device_lds_limit();
 // Skinny MFMA GEMM (qgemm_skinny.hip): any M in blocks of up to 32 rows, the weights streamed
 // once per block.  It takes no workspace.
 hipError_t launch_skinny(const RunArgs& a, hipStream_t s);
-// Up to 4 weights of one quant type and K sharing x and M in one launch (skinny_fits each);
+// Up to 4 weights of one quant type and K sharing x and M in one launch (skinny_group_fits);
 // equal to separate launches bit for bit.
 hipError_t launch_skinny_grouped(const RunArgs* const* items, int n, hipStream_t s);
 // Estimated time of such a launch for M > 32, in microseconds.
@@ -85,8 +85,10 @@ double skinny_est_us(const RunArgs* const* items, int n);
 // How many weight tiles a wavefront of the skinny kernel takes: 1 chosen by shape (default),
 // 0 one, 2 two, 4 four (test hook mlxr_qgemm_test_skinny_stage).
 extern std::atomic<int> g_skinny_stage;
-// Whether every operand of a is below operand_limit() (else: launch_mfma, which chunks).
+// Whether every operand of a is below operand_limit() and the launch's items are countable (else:
+// launch_mfma, which chunks); of a launch of n weights.
 bool skinny_fits(const RunArgs& a);
+bool skinny_group_fits(const RunArgs* const* items, int n);
 // Workspace bytes reported for shapes of the skinny kernel (0: none).
 size_t skinny_workspace_bytes(int M, int N, int K, int qtype);
 // Estimates in microseconds that decide which kernel's workspace size is reported for 32 < M

@@ -667,14 +667,30 @@ size_t skinny_swiglu_workspace_bytes(int M, int N, int K) {
   return pl.ks > 1 ? (size_t)pl.ks * (size_t)M * (size_t)N * 8u : 0;
 }
 
+namespace {
+// The kernel divides an item by the blocks of M with a multiplication (mdiv), which is exact while
+// items x blocks is below 2^32; one tile per wavefront has the most items.
+bool items_fit(int64_t slabs, int M) {
+  const uint64_t mb = ((uint64_t)M + 31) / 32;
+  return (uint64_t)slabs * mb * mb < (1ull << 32);
+}
+}  // namespace
+
 bool skinny_fits(const RunArgs& a) {
   const size_t lim = operand_limit();
   if ((size_t)a.M * (size_t)a.L.K * 2u >= lim) return false;
   for (int i = 0; i < a.L.nplanes; ++i)
     if (a.L.size[i] >= lim) return false;
-  // item / mblocks by a multiplication is exact (any M <= 256; the forced kernel takes larger)
-  const uint64_t mb = ((uint64_t)a.M + 31) / 32;
-  return (uint64_t)((a.L.N + 15) / 16) * mb * mb < (1ull << 32);
+  return items_fit((a.L.N + 15) / 16, a.M);
+}
+
+bool skinny_group_fits(const RunArgs* const* items, int n) {
+  int64_t slabs = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!skinny_fits(*items[i])) return false;
+    slabs += (items[i]->L.N + 15) / 16;
+  }
+  return items_fit(slabs, items[0]->M);
 }
 
 double skinny_mb_est_us(int M, int N, int K) {

@@ -56,3 +56,22 @@ def test_grouped_without_workspace_takes_kernels_of_single_calls(g):
             together = [j for j in range(len(kernels)) if launches[j] == launches[i]]
             assert len(together) <= 4
             assert {(kernels[j], GROUPS[g][j][0]) for j in together} == {(kernels[i], GROUPS[g][i][0])}, M
+
+
+def test_skinny_launch_counts_the_items_of_all_its_weights():
+    """The skinny kernel finds an item's slab by a multiplication that is exact for fewer than 2^32 /
+    blocks of M items: weights that are within it alone and past it together do not share a
+    launch (the quotient of the last items would be wrong, as it is here for two of them)."""
+    M, N, K, blocks = 2000, 12_000_000, 32, 63
+    mdiv = -(-2**32 // blocks)
+    last = lambda n: n * (N // 16) - 1  # the last slab of n weights
+    assert ((last(1) * blocks + blocks - 1) * mdiv) >> 32 == last(1)
+    assert ((last(2) * blocks + blocks - 1) * mdiv) >> 32 != last(2)
+    try:
+        qgemm.test_force_skinny(True)
+        for nbytes in (0, 1 << 40):
+            kernels, launches = qgemm.test_kernels("grouped", [(Q40, N, K)] * 4, M, nbytes)
+            assert kernels != [qgemm.KERNEL_SKINNY] * 4 or len(set(launches)) == 4
+            assert qgemm.test_kernels("grouped", [(Q40, N // 4, K)] * 4, M, nbytes) == ([qgemm.KERNEL_SKINNY] * 4, [0] * 4)
+    finally:
+        qgemm.test_force_skinny(False)
