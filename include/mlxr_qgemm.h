@@ -196,13 +196,14 @@ typedef struct mlxr_qgemm_item {
  * and, for prefill, to fill the device with the small projections' tiles. */
 int mlxr_qgemm_run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,
                            void* stream);
-/* mlxr_qgemm_run_grouped with a caller-owned device workspace (NULL or too small = as
- * mlxr_qgemm_run_grouped).  With it, launches at 32 < M <= 2048 go to the skinny or the
- * tiled kernel, whichever is estimated faster for the weights together, the tiled launches split
- * K over the concatenated N of their weights when their tiles cannot fill the device, and single
- * items run as mlxr_qgemm_run_ws.  Results then differ from separate calls only in
- * fp32 summation order (within the matmul tolerance) and are deterministic for a given
- * (items, M, workspace size).  Same workspace rules as mlxr_qgemm_run_ws. */
+/* mlxr_qgemm_run_grouped with a caller-owned device workspace of the size that
+ * mlxr_qgemm_grouped_workspace_size reports (NULL or less = as mlxr_qgemm_run_grouped; a size of 0
+ * needs none).  With it, launches at 32 < M <= 2048 go to the skinny or the tiled kernel, whichever
+ * is estimated faster for the weights together, the tiled launches split K over the concatenated
+ * N of their weights when their tiles cannot fill the device, and single items run as
+ * mlxr_qgemm_run_ws.  Results then differ from separate calls only in fp32 summation order
+ * (within the matmul tolerance) and are deterministic for a given (items, M, workspace size).
+ * Same workspace rules as mlxr_qgemm_run_ws. */
 int mlxr_qgemm_run_grouped_ws(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,
                               void* workspace_dev, size_t workspace_bytes, void* stream);
 /* Workspace bytes mlxr_qgemm_run_grouped_ws can use for these items at this M (only the
@@ -279,11 +280,14 @@ int mlxr_qgemm_mlp_status(void* workspace_dev, void* stream);
  * All are process-wide (atomics).
  * mlxr_qgemm_test_kernels launches nothing: it tells which kernel would run each item, and which
  * items share a launch (equal numbers in launches), of call 0 mlxr_qgemm_run_ws for each item,
- * 1 mlxr_qgemm_run_grouped_ws, 2 mlxr_qgemm_swiglu with items[0] as gate and up (count 1), given a
- * workspace of workspace_bytes (0: none).  Only the items' qtype, N and K are read. */
+ * 1 mlxr_qgemm_run_grouped_ws, 2 mlxr_qgemm_swiglu with items[0] as gate and up (count 1), 3
+ * mlxr_qgemm_run_grouped, given a workspace of workspace_bytes (0: none).  Only the items' qtype, N and K are read. */
 enum { MLXR_KERNEL_GEMV = 0, MLXR_KERNEL_SKINNY = 1, MLXR_KERNEL_TILED = 2, MLXR_KERNEL_TILED_SPLIT = 3 };
 int mlxr_qgemm_test_kernels(int call, int count, const mlxr_qgemm_item* items, int M, size_t workspace_bytes,
                             int* kernels, int* launches);
+/* The layout of a launch of the skinny kernel: layout[0] weight tiles per wavefront, [1] wavefronts per
+ * workgroup, [2] splits of K over workgroups. */
+int mlxr_qgemm_test_skinny_layout(int qtype, int N, int K, int M, int swiglu, size_t workspace_bytes, int* layout);
 int mlxr_qgemm_test_force_tiled(int on);
 int mlxr_qgemm_test_set_operand_limit(size_t bytes);
 int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks);

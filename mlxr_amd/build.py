@@ -19,8 +19,9 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 # longest compiles first (the pool starts them first)
 SOURCES = ["qgemm_gemv.hip", "qgemm_mlp.hip", "qgemm_tile_q4k.hip", "qgemm_tile_q6k.hip", "qgemm_tile_q5k.hip",
-           "qgemm_tile_q40.hip", "qgemm_tile_q41.hip", "qgemm_tile_q80.hip", "qgemm_skinny.hip",
-           "qgemm_tile.hip", "qgemm_api.hip", "qgemm_pack.hip", "qgemm_noalloc.hip",
+           "qgemm_skinny_q6k.hip", "qgemm_skinny_q80.hip", "qgemm_skinny_q5k.hip", "qgemm_skinny_q4k.hip",
+           "qgemm_skinny_q41.hip", "qgemm_skinny_q40.hip", "qgemm_tile_q40.hip", "qgemm_tile_q41.hip",
+           "qgemm_tile_q80.hip", "qgemm_skinny.hip", "qgemm_tile.hip", "qgemm_api.hip", "qgemm_pack.hip", "qgemm_noalloc.hip",
            "q_gemm_dequant_primitive.cpp", "synth.cpp", "gguf.cpp", "act.hip", "linear.cpp"]
 BENCH_SOURCES = ["bench_probe.hip"]
 COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-Wall",

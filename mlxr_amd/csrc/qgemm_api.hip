@@ -52,7 +52,7 @@ constexpr int kSkinnyMaxM = 2048;
 constexpr int kSizedMaxM = 256;
 bool mid_sized_skinny(int M, const mlxr::PackedLayout& L) {
   if (M > kSizedMaxM) return false;
-  return mlxr::skinny_mb_est_us(M, L.N, L.K) < mlxr::mfma_est_us(M, L.N, L.K, L.qtype, ~(size_t)0);
+  return mlxr::skinny_sizing_us(M, L.N, L.K) < mlxr::mfma_sizing_us(M, L.N, L.K, L.qtype);
 }
 size_t single_workspace(int M, const mlxr::PackedLayout& L) {
   const bool skinny = M <= kSkinnyOnlyMaxM ? !gemv_auto(M, L) : mid_sized_skinny(M, L);
@@ -63,6 +63,15 @@ size_t single_workspace(int M, const mlxr::PackedLayout& L) {
 enum Forced { kNotForced, kForceSkinny, kForceTiled };
 std::atomic<int> g_forced{kNotForced};
 int forced() { return g_forced.load(std::memory_order_relaxed); }
+
+// Whether the skinny kernel is estimated to be ahead of the tiled one, which takes the weights as one
+// of `cols` columns with a workspace of ws_bytes.  The estimates are 7% off on average: where
+// they are within 5% of each other the tiled kernel stays (Q4_K SwiGLU 8192 x 3072 at M = 64, us,
+// skinny / tiled: estimated 24.9 / 25.5, measured 27.2 / 24.2).
+bool skinny_ahead(const mlxr::RunArgs* const* items, int n, bool swiglu, int cols, size_t ws_bytes) {
+  const mlxr::RunArgs& a = *items[0];
+  return mlxr::skinny_us(items, n, swiglu) < 0.95 * mlxr::mfma_us(a.M, cols, a.L.K, a.L.qtype, ws_bytes);
+}
 
 // The kernel of a single call: GEMV (no MFMA) for decode (gemv_auto); MFMA kernels otherwise, the
 // skinny one up to M = 32, then up to M = 2048 the skinny or the tiled one, the tiled one above
@@ -75,27 +84,21 @@ Kernel single_kernel(mlxr::RunArgs& a, int path) {
   if (path == MLXR_PATH_GEMV || (path == MLXR_PATH_AUTO && gemv_auto(M, a.L))) return kGemv;
   const bool fits = mlxr::skinny_fits(a);
   if (forced() != kNotForced) return forced() == kForceSkinny && fits ? kSkinny : kTiled;
-  if (M <= kSkinnyOnlyMaxM) return fits ? kSkinny : kTiled;
   if (M > kSkinnyMaxM) return kTiled;
-  // a workspace below the size mlxr_qgemm_workspace_size asks for is not used; a call
-  // whose size is 0 has what it asks for, with or without one
+  // a workspace below the size mlxr_qgemm_workspace_size asks for is not used, and no more than
+  // that of a larger one; a call whose size is 0 has what it asks for, with or without one
   const size_t need = single_workspace(M, a.L);
   const bool ws_ok = need == 0 || (a.ws && a.ws_bytes >= need);
-  if (!ws_ok && M <= kSizedMaxM) {
-    a.ws = nullptr;
-    a.ws_bytes = 0;
-  }
+  if (need == 0 || (!ws_ok && M <= kSizedMaxM)) a.ws = nullptr;
+  a.ws_bytes = a.ws ? std::min(a.ws_bytes, need) : 0;
   if (!fits) return kTiled;
-  // with it, the tiled kernel runs where its size was reported and it is estimated to be
-  // ahead (4096 x 4096 Q4_K, us, tiled / skinny: M = 64 18.1 / 10.7, M = 128 23.7 / 14.4, M =
-  // 256 26.9 / 24.6; 14336 x 4096: M = 64 25.9 / 26.2, M = 128 33.4 / 47.6); without, the
-  // skinny one takes M <= 64 and the tiled one (unsplit) larger M
+  if (M <= kSkinnyOnlyMaxM) return kSkinny;
+  // by the estimates (4096 x 4096 Q4_K, us, tiled / skinny: M = 64 18.1 / 10.7, M = 128 23.7 / 14.4, M
+  // = 256 26.9 / 24.6; 14336 x 4096: M = 64 25.9 / 26.2, M = 128 33.4 / 47.6); without the workspace
+  // asked for, the skinny one takes M <= 64 and the tiled one (unsplit) larger M
   if (!ws_ok) return M <= 64 ? kSkinny : kTiled;
   const mlxr::RunArgs* one[1] = {&a};
-  return mid_sized_skinny(M, a.L) ||
-                 mlxr::skinny_est_us(one, 1) < mlxr::mfma_est_us(M, a.L.N, a.L.K, a.L.qtype, ~(size_t)0)
-             ? kSkinny
-             : kTiled;
+  return skinny_ahead(one, 1, false, a.L.N, a.ws_bytes) ? kSkinny : kTiled;
 }
 
 thread_local std::string g_err;
@@ -412,7 +415,7 @@ bool batch_skinny(const mlxr::RunArgs* const* items, int n, int M, size_t ws_byt
     cols += items[i]->L.N;
   }
   if (forced() == kForceSkinny) return true;
-  return mlxr::skinny_est_us(items, n) < mlxr::mfma_est_us(M, cols, items[0]->L.K, items[0]->L.qtype, ws_bytes);
+  return skinny_ahead(items, n, false, cols, ws_bytes);
 }
 
 // The workspace reported for a grouped call.
@@ -429,19 +432,19 @@ size_t grouped_need(const std::vector<mlxr::RunArgs>& a, int M) {
   return need;
 }
 
-// The batches of a call and their kernels (kGroupedTiled / kGroupedSkinny decided).  A workspace
-// below the reported size is none, and so is one of a call whose size is 0: *ws is cleared.
-std::vector<Batch> call_batches(const std::vector<mlxr::RunArgs>& a, int M, void** ws, size_t ws_bytes) {
-  if (*ws) {
-    const size_t need = grouped_need(a, M);
-    if (need == 0 || ws_bytes < need) *ws = nullptr;
-  }
-  std::vector<Batch> out = plan_batches(a, M, *ws != nullptr, false);
+// The batches of a call and their kernels (kGroupedTiled / kGroupedSkinny decided).  sized: the call
+// takes a workspace; one below the reported size is none and *ws is cleared, a size of 0 asks for
+// none.
+std::vector<Batch> call_batches(const std::vector<mlxr::RunArgs>& a, int M, bool sized, void** ws, size_t ws_bytes) {
+  const size_t need = sized ? grouped_need(a, M) : 1;
+  if (need == 0 || !*ws || ws_bytes < need) *ws = nullptr;
+  const bool have = need == 0 || *ws;
+  std::vector<Batch> out = plan_batches(a, M, have, false);
   for (Batch& bt : out) {
-    if (bt.kind != kGroupedTiled || !*ws) continue;
+    if (bt.kind != kGroupedTiled || !have) continue;
     const mlxr::RunArgs* batch[4];
     for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
-    if (batch_skinny(batch, bt.n, M, ws_bytes)) bt.kind = kGroupedSkinny;
+    if (batch_skinny(batch, bt.n, M, *ws ? ws_bytes : 0)) bt.kind = kGroupedSkinny;
   }
   return out;
 }
@@ -481,13 +484,13 @@ int grouped_args(int count, const mlxr_qgemm_item* items, const void* x_dev, int
   return MLXR_OK;
 }
 
-int run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M, void* ws,
+int run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M, bool sized, void* ws,
                 size_t ws_bytes, void* stream) {
   std::vector<mlxr::RunArgs> a;
   int rc = grouped_args(count, items, x_dev, x_dtype, M, true, stream, a);
   if (rc || count == 0 || M == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
-  for (const Batch& bt : call_batches(a, M, &ws, ws_bytes)) {
+  for (const Batch& bt : call_batches(a, M, sized, &ws, ws_bytes)) {
     const mlxr::RunArgs* batch[4];
     for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
     if (bt.kind == kGroupedGemv) {
@@ -515,12 +518,12 @@ extern "C" {
 
 int mlxr_qgemm_run_grouped(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,
                            void* stream) {
-  return run_grouped(count, items, x_dev, x_dtype, M, nullptr, 0, stream);
+  return run_grouped(count, items, x_dev, x_dtype, M, false, nullptr, 0, stream);
 }
 
 int mlxr_qgemm_run_grouped_ws(int count, const mlxr_qgemm_item* items, const void* x_dev, int x_dtype, int M,
                               void* workspace_dev, size_t workspace_bytes, void* stream) {
-  return run_grouped(count, items, x_dev, x_dtype, M, workspace_dev, workspace_dev ? workspace_bytes : 0, stream);
+  return run_grouped(count, items, x_dev, x_dtype, M, true, workspace_dev, workspace_dev ? workspace_bytes : 0, stream);
 }
 
 int mlxr_qgemm_grouped_workspace_size(int count, const mlxr_qgemm_item* items, int M, size_t* bytes) {
@@ -549,13 +552,13 @@ int swiglu_kind(const mlxr::RunArgs& a) {
 // (5632 x 2048 Q4_K at M = 64, us, tiled / skinny: 19.9 / 16.2).  ws: the call has the workspace
 // that its size asks for.
 int swiglu_kernel(const mlxr::RunArgs& g, const mlxr::RunArgs& u, bool ws) {
-  const int kind = swiglu_kind(g), M = g.M, N = g.L.N, K = g.L.K;
+  const int kind = swiglu_kind(g), M = g.M, N = g.L.N;
   if (kind == 0 || kind == 3) return kind;
   if (forced() != kNotForced) return forced() == kForceTiled ? 2 : mlxr::skinny_fits(g) ? 1 : 2;
   if (kind == 1 || M > kSkinnyMaxM || !mlxr::skinny_fits(g) || N > INT32_MAX / 2) return kind;
   const mlxr::RunArgs* both[2] = {&g, &u};
   const size_t have = ws ? ~(size_t)0 : 0;
-  return mlxr::skinny_est_us(both, 2) < mlxr::mfma_est_us(M, 2 * N, K, g.L.qtype, have) ? 1 : 2;
+  return skinny_ahead(both, 2, true, 2 * N, have) ? 1 : 2;
 }
 }  // namespace
 
@@ -613,7 +616,7 @@ int mlxr_qgemm_swiglu(int qtype, int N, int K, const void* gate_packed, const vo
     // a workspace smaller than the split plan's runs the launch unsplit
     void* ws = workspace_dev && workspace_bytes >= need ? workspace_dev : nullptr;
     g.ws = ws;
-    g.ws_bytes = ws ? workspace_bytes : 0;
+    g.ws_bytes = ws ? need : 0;
     const hipError_t e =
         kind == 1 ? mlxr::launch_skinny_swiglu(g, u, s) : mlxr::launch_mfma_swiglu(g, u, ws, g.ws_bytes, s);
     return e != hipSuccess ? hip_fail(e, "swiglu launch") : MLXR_OK;
@@ -778,7 +781,7 @@ int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks) {
 }
 
 int mlxr_qgemm_test_skinny_stage(int on) {
-  mlxr::g_skinny_stage.store(on <= 0 ? 0 : on >= 3 ? 4 : on, std::memory_order_relaxed);
+  mlxr::g_skinny_tiles.store(on <= 0 ? 1 : on == 1 ? 0 : on == 2 ? 2 : 4, std::memory_order_relaxed);
   return MLXR_OK;
 }
 
@@ -794,7 +797,7 @@ int mlxr_qgemm_test_force_tiled(int on) {
 
 int mlxr_qgemm_test_kernels(int call, int count, const mlxr_qgemm_item* items, int M, size_t workspace_bytes,
                             int* kernels, int* launches) {
-  if (call < 0 || call > 2 || (call == 2 && count != 1) || !kernels || !launches || M < 1)
+  if (call < 0 || call > 3 || (call == 2 && count != 1) || !kernels || !launches || M < 1)
     return fail(MLXR_E_INVALID, "invalid kernel query");
   std::vector<mlxr::RunArgs> a;
   const int rc = grouped_args(count, items, nullptr, MLXR_BF16, M, false, nullptr, a);
@@ -814,10 +817,10 @@ int mlxr_qgemm_test_kernels(int call, int count, const mlxr_qgemm_item* items, i
       kernels[i] = single(i);
       launches[i] = i;
     }
-  } else if (call == 1) {
-    void* gws = ws;
+  } else if (call == 1 || call == 3) {
+    void* gws = call == 1 ? ws : nullptr;
     int launch = 0;
-    for (const Batch& bt : call_batches(a, M, &gws, workspace_bytes)) {
+    for (const Batch& bt : call_batches(a, M, call == 1, &gws, workspace_bytes)) {
       const mlxr::RunArgs* batch[4];
       for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
       const bool split = bt.kind == kGroupedTiled && gws && mlxr::mfma_grouped_workspace_bytes(batch, bt.n) > 0;
@@ -845,6 +848,20 @@ int mlxr_qgemm_test_kernels(int call, int count, const mlxr_qgemm_item* items, i
                      : MLXR_KERNEL_TILED;
     launches[0] = 0;
   }
+  return MLXR_OK;
+}
+
+int mlxr_qgemm_test_skinny_layout(int qtype, int N, int K, int M, int swiglu, size_t workspace_bytes, int* layout) {
+  mlxr::RunArgs a;
+  const int rc = check_type_shape(qtype, N, K, &a.L);
+  if (rc) return rc;
+  if (!layout || M < 1) return fail(MLXR_E_INVALID, "invalid layout query");
+  a.x_dtype = MLXR_BF16;
+  a.M = M;
+  a.ws = workspace_bytes ? (void*)layout : nullptr;  // only compared with null
+  a.ws_bytes = workspace_bytes;
+  const mlxr::RunArgs* items[2] = {&a, &a};
+  mlxr::skinny_layout(items, swiglu ? 2 : 1, swiglu != 0, layout);
   return MLXR_OK;
 }
 

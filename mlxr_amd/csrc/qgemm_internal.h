@@ -80,21 +80,26 @@ hipError_t launch_skinny(const RunArgs& a, hipStream_t s);
 // Up to 4 weights of one quant type and K sharing x and M in one launch (skinny_group_fits);
 // equal to separate launches bit for bit.
 hipError_t launch_skinny_grouped(const RunArgs* const* items, int n, hipStream_t s);
-// Estimated time of such a launch for M > 32, in microseconds.
-double skinny_est_us(const RunArgs* const* items, int n);
-// How many weight tiles a wavefront of the skinny kernel takes: 1 chosen by shape (default),
-// 0 one, 2 two, 4 four (test hook mlxr_qgemm_test_skinny_stage).
-extern std::atomic<int> g_skinny_stage;
+// Estimated time of such a launch in microseconds (swiglu: of launch_skinny_swiglu).
+double skinny_us(const RunArgs* const* items, int n, bool swiglu);
+// Its weight tiles per wavefront, wavefronts per workgroup and splits of K over workgroups.
+void skinny_layout(const RunArgs* const* items, int n, bool swiglu, int* layout);
+// What tests force on the skinny kernel, 0 by shape (default): weight tiles of a wavefront (1, 2, 4;
+// SwiGLU 2, 4).
+extern std::atomic<int> g_skinny_tiles;
 // Whether every operand of a is below operand_limit() and the launch's items are countable (else:
 // launch_mfma, which chunks); of a launch of n weights.
 bool skinny_fits(const RunArgs& a);
 bool skinny_group_fits(const RunArgs* const* items, int n);
 // Workspace bytes reported for shapes of the skinny kernel (0: none).
 size_t skinny_workspace_bytes(int M, int N, int K, int qtype);
-// Estimates in microseconds that decide which kernel's workspace size is reported for 32 < M
-// <= 256: a skinny kernel in 64-row blocks, and launch_mfma with a workspace of ws_bytes.
-double skinny_mb_est_us(int M, int N, int K);
-double mfma_est_us(int M, int N, int K, int qtype, size_t ws_bytes);
+// Which kernel's workspace size is reported for 32 < M <= 256 is decided by two estimates, fixed
+// because callers size their buffers by the result; they choose no kernel.
+double skinny_sizing_us(int M, int N, int K);
+double mfma_sizing_us(int M, int N, int K, int qtype);
+// Estimated time in microseconds of the tiled kernel over an [M, N, K] problem that has a workspace
+// of ws_bytes, of its launch and the reduce.
+double mfma_us(int M, int N, int K, int qtype, size_t ws_bytes);
 // SwiGLU, h = swish(x.gate^T + bias_g) * (x.up^T + bias_u) into gate.y, with gate and up
 // of one type and shape; gate.ws / ws (may be null) holds split-K partials.
 // Skinny kernel and tiled kernel (any M; operands below 2 GiB, mfma_groupable; no biases).

@@ -1,0 +1,13 @@
+// Instantiates the skinny kernel (qgemm_skinny_kernel.h) for Q4_0 weights; one translation unit
+// per quant type keeps the build parallel.
+#include "qgemm_skinny_kernel.h"
+
+namespace mlxr {
+namespace skinny {
+
+const SkinnyKern& kern_q40(bool f16, int xr, int rt, bool sw) {
+  return f16 ? kern_of<QT_Q4_0, X_F16>(xr, rt, sw) : kern_of<QT_Q4_0, X_BF16>(xr, rt, sw);
+}
+
+}  // namespace skinny
+}  // namespace mlxr

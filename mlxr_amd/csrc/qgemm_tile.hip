@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -459,8 +460,8 @@ hipError_t launch_splitk_reduce_swiglu(const float* ws, size_t split_elems, int 
   return hipGetLastError();
 }
 
-double mfma_est_us(int M, int N, int K, int qtype, size_t ws_bytes) {
-  const SplitPlan sp = plan_split(M, N, K, ws_bytes);
+double mfma_sizing_us(int M, int N, int K, int qtype) {
+  const SplitPlan sp = plan_split(M, N, K, ~(size_t)0);
   const int nkt = (K + TK - 1) / TK;
   const long rounds = ((long)sp.tiles * sp.S + device_cu_count() - 1) / device_cu_count();
   // Q6_K steps dequantize more per weight: measured on MI355X (Llama-3-70B v, 1024x8192,
@@ -471,6 +472,31 @@ double mfma_est_us(int M, int N, int K, int qtype, size_t ws_bytes) {
   // launches of one ring per workgroup take about 4.5 us more than the model says
   // (measured on MI355X, Llama-3-8B q/k shapes at M = 64-512)
   return t * 1.86 + (sp.kps <= 8 && nkt > 8 ? 4.5 : 0.0);
+}
+
+// Measured on MI355X over 21 shapes of ordinary models at M = 33 .. 2048, all types, split and
+// not, SwiGLU as 2N columns (7% off on average): us of a step of 256-, 128- and 64-row tiles, Q4_K,
+// and what the other types' dequantization makes of it (past the first steps, which wait for memory); 8 us per round of workgroups beside its
+// steps, of which a round that fills a part of the CUs saves a sixth of the empty part; the reduce
+// launch.
+double mfma_us(int M, int N, int K, int qtype, size_t ws_bytes) {
+  SplitPlan sp = plan_split(M, N, K, ~(size_t)0);
+  if (sp.S > 1 && (size_t)sp.S * (size_t)M * (size_t)N * 4u > ws_bytes) sp = plan_split(M, N, K, 0);
+  constexpr double kStep[3] = {1.55, 0.89, 0.66};
+  static const double kType[4][3] = {{1, 1, 1}, {1.13, 1.28, 1.46}, {1.17, 1.32, 1.52}, {1.11, 1.30, 1.55}};
+  const int b = sp.bm == 256 ? 0 : sp.bm == 128 ? 1 : 2;
+  const int t = qtype == QT_Q5_K ? 1 : qtype == QT_Q6_K ? 2 : qtype == QT_Q8_0 ? 3 : 0;
+  const double q4 = qtype == QT_Q4_0 || qtype == QT_Q4_1 ? 1.0 + 0.06 * b : 1.0;
+  const int cus = device_cu_count(), ring = qtype == QT_Q8_0 ? 4 : 8;
+  const int steps = ((sp.S > 1 ? sp.kps : (K + TK - 1) / TK) + ring - 1) / ring * ring;
+  const long wgs = (long)sp.tiles * sp.S;
+  const double part = (double)(wgs % cus) / cus;
+  const double round = steps * kStep[b] + std::max(steps - 6, 0) * kStep[b] * (kType[t][b] * q4 - 1.0) + 8.0;
+  double us = (wgs / cus + (part > 0 ? 0.84 + 0.16 * part : 0)) * round;
+  if (sp.S > 1) us += 3.8 + (double)sp.S * M * N * 8.0 / 6.4e6;
+  // operands at 3 TB/s
+  const double m = ((double)N * K * gguf_block_bytes(qtype) / gguf_block_elems(qtype) + 2.0 * M * ((double)N + K)) / 3e6;
+  return std::sqrt(std::sqrt(us * us * us * us + m * m * m * m));
 }
 
 size_t mfma_workspace_bytes(int M, int N, int K) {

@@ -89,6 +89,7 @@ _SIGS = {
     "mlxr_qgemm_test_force_skinny": (ctypes.c_int, [ctypes.c_int]),
     "mlxr_qgemm_test_force_tiled": (ctypes.c_int, [ctypes.c_int]),
     "mlxr_qgemm_test_kernels": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_void_p]),
+    "mlxr_qgemm_test_skinny_layout": (ctypes.c_int, [ctypes.c_int] * 5 + [ctypes.c_size_t, ctypes.c_void_p]),
     "mlxr_qgemm_test_skinny_stage": (ctypes.c_int, [ctypes.c_int]),
     "mlxr_qgemm_auto_path": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                              ctypes.POINTER(ctypes.c_int)]),
@@ -456,12 +457,13 @@ KERNEL_GEMV, KERNEL_SKINNY, KERNEL_TILED, KERNEL_TILED_SPLIT = 0, 1, 2, 3
 
 def test_kernels(call, weights, M, workspace_bytes=0):
     """Test hook: the kernel (KERNEL_*) of each (qtype, N, K) of `weights`, and the number of the launch
-    it is part of, for call "single", "grouped" or "swiglu" with a workspace of that size.
+    it is part of, for call "single", "grouped_ws", "swiglu" or "grouped" with a workspace of that
+    size.
     Launches nothing."""
     n = len(weights)
     arr = (Item * n)(*[Item(int(qt), N, K, 0, None, None, F32, None, F32) for qt, N, K in weights])
     kernels, launches = (ctypes.c_int * n)(), (ctypes.c_int * n)()
-    _check(lib().mlxr_qgemm_test_kernels({"single": 0, "grouped": 1, "swiglu": 2}[call], n, arr, int(M),
+    _check(lib().mlxr_qgemm_test_kernels({"single": 0, "grouped_ws": 1, "swiglu": 2, "grouped": 3}[call], n, arr, int(M),
                                          int(workspace_bytes), kernels, launches))
     return list(kernels), list(launches)
 
@@ -470,3 +472,10 @@ def test_skinny_stage(mode):
     """Test hook: weight tiles a wavefront of the skinny kernel takes: 0 (False) one, 2 two,
     3 and above four (SwiGLU: two, two, four); 1 (True, the default) chooses by shape."""
     _check(lib().mlxr_qgemm_test_skinny_stage(int(mode)))
+
+
+def test_skinny_layout(qtype, N, K, M, swiglu=False, workspace_bytes=0):
+    """Test hook: (tiles per wavefront, wavefronts, splits of K) of a launch of the skinny kernel."""
+    v = (ctypes.c_int * 3)()
+    _check(lib().mlxr_qgemm_test_skinny_layout(int(qtype), N, K, M, 1 if swiglu else 0, int(workspace_bytes), v))
+    return tuple(v)
