@@ -276,7 +276,9 @@ int mlxr_qgemm_mlp_status(void* workspace_dev, void* stream);
  * tiled kernel (split over K where the call's workspace holds its partials).
  * mlxr_qgemm_test_skinny_stage: weight tiles a wavefront of
  * the skinny kernel takes: 0 one, 2 two, 3 and above four (SwiGLU: two, two, four), 1 restores
- * the choice by shape; tests use it to check every variant against the oracle.
+ * the choice by shape; mlxr_qgemm_test_skinny_plan sets them too (1, 2, 4), with the wavefronts of a
+ * workgroup (8, or 1 where K <= 1024), each 0 by shape; tests use them to check every variant
+ * against the oracle.
  * All are process-wide (atomics).
  * mlxr_qgemm_test_kernels launches nothing: it tells which kernel would run each item, and which
  * items share a launch (equal numbers in launches), of call 0 mlxr_qgemm_run_ws for each item,
@@ -293,6 +295,7 @@ int mlxr_qgemm_test_set_operand_limit(size_t bytes);
 int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks);
 int mlxr_qgemm_test_force_skinny(int on);
 int mlxr_qgemm_test_skinny_stage(int on);
+int mlxr_qgemm_test_skinny_plan(int tiles, int waves);
 
 /* Deterministic synthetic inputs with the shapes/distributions of the benchmark
  * configurations (host memory).  Generator: SplitMix64 from `seed`; normals by

@@ -781,7 +781,14 @@ int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks) {
 }
 
 int mlxr_qgemm_test_skinny_stage(int on) {
-  mlxr::g_skinny_tiles.store(on <= 0 ? 1 : on == 1 ? 0 : on == 2 ? 2 : 4, std::memory_order_relaxed);
+  return mlxr_qgemm_test_skinny_plan(on <= 0 ? 1 : on == 1 ? 0 : on == 2 ? 2 : 4, 0);
+}
+
+int mlxr_qgemm_test_skinny_plan(int tiles, int waves) {
+  if ((tiles != 0 && tiles != 1 && tiles != 2 && tiles != 4) || (waves != 0 && waves != 1 && waves != 8))
+    return fail(MLXR_E_INVALID, "invalid skinny plan");
+  mlxr::g_skinny_tiles.store(tiles, std::memory_order_relaxed);
+  mlxr::g_skinny_waves.store(waves, std::memory_order_relaxed);
   return MLXR_OK;
 }
 

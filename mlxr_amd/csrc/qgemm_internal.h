@@ -85,8 +85,8 @@ double skinny_us(const RunArgs* const* items, int n, bool swiglu);
 // Its weight tiles per wavefront, wavefronts per workgroup and splits of K over workgroups.
 void skinny_layout(const RunArgs* const* items, int n, bool swiglu, int* layout);
 // What tests force on the skinny kernel, 0 by shape (default): weight tiles of a wavefront (1, 2, 4;
-// SwiGLU 2, 4).
-extern std::atomic<int> g_skinny_tiles;
+// SwiGLU 2, 4), wavefronts of a workgroup (1, 8).
+extern std::atomic<int> g_skinny_tiles, g_skinny_waves;
 // Whether every operand of a is below operand_limit() and the launch's items are countable (else:
 // launch_mfma, which chunks); of a launch of n weights.
 bool skinny_fits(const RunArgs& a);

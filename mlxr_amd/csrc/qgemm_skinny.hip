@@ -10,20 +10,20 @@
 
 namespace mlxr {
 
-std::atomic<int> g_skinny_tiles{0};
+std::atomic<int> g_skinny_tiles{0}, g_skinny_waves{0};
 
 namespace {
 
 using namespace skinny;
 
-const SkinnyKern& kern_for(int qtype, bool f16, int xr, int rt, bool sw) {
+const SkinnyKern& kern_for(int qtype, bool f16, int xr, int rt, int kg, bool sw) {
   switch (qtype) {
-    case QT_Q4_K: return kern_q4k(f16, xr, rt, sw);
-    case QT_Q6_K: return kern_q6k(f16, xr, rt, sw);
-    case QT_Q5_K: return kern_q5k(f16, xr, rt, sw);
-    case QT_Q4_0: return kern_q40(f16, xr, rt, sw);
-    case QT_Q4_1: return kern_q41(f16, xr, rt, sw);
-    default: return kern_q80(f16, xr, rt, sw);
+    case QT_Q4_K: return kern_q4k(f16, xr, rt, kg, sw);
+    case QT_Q6_K: return kern_q6k(f16, xr, rt, kg, sw);
+    case QT_Q5_K: return kern_q5k(f16, xr, rt, kg, sw);
+    case QT_Q4_0: return kern_q40(f16, xr, rt, kg, sw);
+    case QT_Q4_1: return kern_q41(f16, xr, rt, kg, sw);
+    default: return kern_q80(f16, xr, rt, kg, sw);
   }
 }
 
@@ -46,9 +46,10 @@ int residents(const SkinnyKern& k, hipError_t* e) {
   return occ;
 }
 
-// How a launch is laid out: weight tiles of a wavefront, and its estimated time.
+// How a launch is laid out: weight tiles of a wavefront, wavefronts of a workgroup (8, or 1 for short
+// K), and its estimated time.
 struct Plan {
-  int rt;
+  int rt, kg;
   double us;
 };
 
@@ -56,28 +57,31 @@ struct Plan {
 // types, weights from memory (7% off on average; the variant chosen by it 0.2% slower than the best
 // one on average, 1% or less for 95%).  us of a turn (one super-block for each of eight
 // wavefronts) of a workgroup, by rows of X (8, 16, 32) and tiles (1, 2, 4), Q4_K; the workgroups of
-// a CU take as many.  The other types by their dequantization.
+// a CU take as many.  A lone wavefront's super-block takes kLoneLat + n * kLoneCu on a CU of n.  The
+// other types by their dequantization.
 constexpr double kTurn[3][3] = {{1.25, 2.31, 4.20}, {1.64, 2.62, 4.52}, {2.32, 3.27, 5.22}};
+constexpr double kLoneLat[3][3] = {{0.63, 1.43, 2.46}, {0.73, 1.47, 2.63}, {0.87, 1.77, 3.14}};
+constexpr double kLoneCu[3][3] = {{0.10, 0.07, 0.26}, {0.12, 0.13, 0.24}, {0.18, 0.20, 0.35}};
 struct TypeCost {
-  double turn[3];
+  double turn[3], lone;
 };
 TypeCost type_cost(int qtype) {
   switch (qtype) {
-    case QT_Q5_K: return {{1.13, 1.23, 1.26}};
-    case QT_Q6_K: return {{1.19, 1.30, 1.35}};
-    case QT_Q8_0: return {{1.11, 1.15, 1.16}};
-    case QT_Q4_0: return {{0.98, 0.99, 1.00}};
-    case QT_Q4_1: return {{0.99, 1.00, 1.01}};
-    default: return {{1.0, 1.0, 1.0}};
+    case QT_Q5_K: return {{1.13, 1.23, 1.26}, 1.19};
+    case QT_Q6_K: return {{1.19, 1.30, 1.35}, 1.22};
+    case QT_Q8_0: return {{1.11, 1.15, 1.16}, 1.02};
+    case QT_Q4_0: return {{0.98, 0.99, 1.00}, 0.94};
+    case QT_Q4_1: return {{0.99, 1.00, 1.01}, 0.95};
+    default: return {{1.0, 1.0, 1.0}, 1.0};
   }
 }
-// What the weights' bytes take, MB/us (TB/s), by tiles.
-constexpr double kBytes[3] = {3.57, 3.76, 3.98};
+// What the weights' bytes take, MB/us (TB/s), by tiles: eight wavefronts, a lone one.
+constexpr double kBytes[2][3] = {{3.57, 3.76, 3.98}, {3.71, 3.30, 4.09}};
 
-// us of a launch of `items` items of `turns` turns, `occ` workgroups on a CU.
+// us of a launch of `items` items of `turns` turns (kg = 1: super-blocks), `occ` workgroups on a CU.
 // Whole rounds of the device's workgroups, then the rest: the first workgroups, neighbours on an
 // XCD, take one item more.  The weights' bytes are read again, half from memory, by further blocks of M.
-double plan_us(int qtype, int xr, int rt, long items, long turns, int occ, int mblocks, double bytes) {
+double plan_us(int qtype, int xr, int rt, int kg, long items, long turns, int occ, int mblocks, double bytes) {
   const int x = xr == 8 ? 0 : xr == 16 ? 1 : 2, t = rt == 1 ? 0 : rt == 2 ? 1 : 2;
   const long cus = device_cu_count(), slots = occ * cus;
   const long full = items / slots, rest = items % slots;
@@ -85,38 +89,47 @@ double plan_us(int qtype, int xr, int rt, long items, long turns, int occ, int m
   const TypeCost tc = type_cost(qtype);
   auto dur = [&](long n) {
     if (n == 0) return 0.0;
-    return turns * kTurn[x][t] * tc.turn[t] * (n + 0.1) / 1.1 + 0.3;
+    return kg == 1 ? turns * (kLoneLat[x][t] + kLoneCu[x][t] * n) * tc.lone
+                   : turns * kTurn[x][t] * tc.turn[t] * (n + 0.1) / 1.1 + 0.3;
   };
-  const double c = 2.6, a = c + full * dur(occ) + dur(n);
-  const double m = c + bytes * (0.5 + 0.5 * mblocks) * 1e-6 / kBytes[t];
+  const double c = kg == 1 ? 2.8 : 2.6;
+  const double a = c + full * dur(occ) + dur(n);
+  const double m = c + bytes * (0.5 + 0.5 * mblocks) * 1e-6 / kBytes[kg == 1][t];
   return std::sqrt(std::sqrt(a * a * a * a + m * m * m * m));
 }
 
 // The plan of a launch: the fastest by plan_us.  (One rule on the items for three quarters of the CUs
 // took two tiles for 5120 rows in two blocks of M, two rounds where four need one: Q4_K 5120 x
 // 13824 at M = 33 47.4 us, at four tiles 36.9.)
+// Eight wavefronts share a K of more than 1024, where the split of K and so the sums depend on K
+// alone.  Up to 1024 each has at most one super-block, a lone wavefront takes them in the same
+// order, and the sums are the same bits: a wide weight then need not meet in LDS once per item
+// (Q4_K 65536 x 1024 at M = 8 20.4 -> 14.0 us, 16384 x 256 7.5 -> 4.2; 1536 x 1024 4.1 with eight
+// wavefronts, 5.7 with one).
 Plan plan_for(const RunArgs* const* items, int n, bool swiglu) {
   const RunArgs& a = *items[0];
   const int M = a.M, K = a.L.K, xr = rows_of_block(M);
   const bool f16 = a.x_dtype == DT_F16;
-  const int tiles = g_skinny_tiles.load(std::memory_order_relaxed), turns = (K + 2047) / 2048;
+  const int tiles = g_skinny_tiles.load(std::memory_order_relaxed), waves = g_skinny_waves.load(std::memory_order_relaxed);
+  const int nsb = (K + 255) / 256, turns = (nsb + 7) / 8;
   double bytes = 0;
   for (int i = 0; i < n; ++i) bytes += (double)items[i]->L.total;
-  Plan best{0, 1e30};
-  auto consider = [&](int rt) {
+  Plan best{0, 0, 1e30};
+  auto consider = [&](int rt, int kg) {
     const int rows = (swiglu ? 8 : 16) * rt;
     long slabs = 0;
     for (int i = 0; i < (swiglu ? 1 : n); ++i) slabs += (items[i]->L.N + rows - 1) / rows;
     hipError_t e;
-    const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, swiglu), &e));
+    const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, kg, swiglu), &e));
     const int mblocks = (M + xr - 1) / xr;
-    const double us = plan_us(a.L.qtype, xr, rt, slabs * mblocks, turns, occ, mblocks, bytes);
-    if (us < best.us) best = Plan{rt, us};
+    const double us = plan_us(a.L.qtype, xr, rt, kg, slabs * mblocks, kg == 1 ? nsb : turns, occ, mblocks, bytes);
+    if (us < best.us) best = Plan{rt, kg, us};
   };
   for (int rt : {1, 2, 4}) {
     if (swiglu && rt == 1) continue;
     if (tiles && rt != (swiglu ? std::max(tiles, 2) : tiles)) continue;
-    consider(rt);
+    if (waves != 1 || K > 1024) consider(rt, 8);
+    if (waves != 8 && K <= 1024) consider(rt, 1);
   }
   return best;
 }
@@ -146,7 +159,7 @@ hipError_t launch_any(const RunArgs* const* items, int n, bool swiglu, hipStream
   sp.ngroups = n;
   sp.parts = (a.M + xr - 1) / xr;
   sp.mdiv = sp.parts > 1 ? (uint32_t)(((1ull << 32) + sp.parts - 1) / sp.parts) : 0u;
-  const SkinnyKern& k = kern_for(a.L.qtype, a.x_dtype == DT_F16, xr, pl.rt, swiglu);
+  const SkinnyKern& k = kern_for(a.L.qtype, a.x_dtype == DT_F16, xr, pl.rt, pl.kg, swiglu);
   hipError_t e = hipSuccess;
   const int occ = residents(k, &e);
   if (occ == 0) return e;
@@ -197,7 +210,7 @@ double skinny_us(const RunArgs* const* items, int n, bool swiglu) { return plan_
 void skinny_layout(const RunArgs* const* items, int n, bool swiglu, int* layout) {
   const Plan pl = plan_for(items, n, swiglu);
   layout[0] = pl.rt;
-  layout[1] = 8;
+  layout[1] = pl.kg;
   layout[2] = 1;
 }
 

@@ -7,13 +7,14 @@
 // weights are its first operand in tiles of 16 rows of N, the activations the second in
 // blocks of 16 rows of M.
 //
-// Work split: a workgroup of NG x KG wavefronts owns a slab of NG * RT * 16 weight rows, for
-// every K.  Wavefront (ng, kg) owns RT tiles of the slab and every KG-th super-block (256 of
-// K), walked in steps of 128: lane (r, j) = (lane % 16, lane / 16) owns sub-block j of the
-// step for row r of each tile, and MFMA kk takes word kk of every lane's sub-block (K
-// positions 32j + 8kk .. +7 of the step, for both operands).  The partial tiles of the KG
-// wavefronts meet in LDS at the end and are added in wavefront order.  The K split depends on
-// K alone, so an output's sum does not depend on how many rows or weights a launch holds.
+// Work split: a workgroup of KG wavefronts owns a slab of RT * 16 weight rows.  Wavefront kg takes
+// every KG-th super-block (256 of K) of its RT tiles, walked in steps of 128: lane (r, j) = (lane %
+// 16, lane / 16) owns sub-block j of the step for row r of each tile, and MFMA kk takes word kk of
+// every lane's sub-block (K positions 32j + 8kk .. +7 of the step, for both operands).  The partial
+// tiles of the KG wavefronts meet in LDS at the end and are added in wavefront order.  KG is 8; a
+// lone wavefront (KG = 1, K <= 1024, where the eight have a super-block or less) adds the same
+// super-blocks in the same order and has neither barrier nor exchange.  So an output's sum does not
+// depend on how many rows or weights a launch holds.
 //
 // The activations go through LDS, read with whole 256-byte row segments.  (Read straight
 // into the operand layout, one load instruction touches 64 different 64-byte segments and
@@ -190,20 +191,22 @@ __device__ __forceinline__ void get_raw(const uint8_t* l, int i, Raw<QT>& r) {
 }
 
 // LDS of a wavefront: activations, two tile slots, headers; the partial tiles reuse it.
-template <int QT, int XR, int RT>
+template <int QT, int XR, int RT, int KG>
 constexpr int wave_lds() {
-  return std::max(XR * 256 + 2 * tile_lds<QT>() + align16(hdr_lds<QT, RT>()), RT * ((XR + 15) / 16) * 1024);
+  constexpr int stage = XR * 256 + 2 * tile_lds<QT>() + align16(hdr_lds<QT, RT>());
+  return KG == 1 ? stage : std::max(stage, RT * ((XR + 15) / 16) * 1024);
 }
 
 // Wavefronts per SIMD the registers are bounded for: 4 (two workgroups on a CU) where that takes
-// no more than a handful of spills, else 2.
-template <int QT, int XR, int RT>
+// no more than a handful of spills, else 2 (lone wavefronts: 3).
+template <int QT, int XR, int RT, int KG>
 constexpr int skinny_occ() {
+  if (KG == 1 && RT == 4 && XR <= 16) return 3;
   return XR > 16 || QT == QT_Q6_K || QT == QT_Q8_0 || (QT == QT_Q5_K && XR == 16 && RT == 4) ? 2 : 4;
 }
 
 template <int QT, int XT, int XR, int RT, int D, int KG, bool SW>
-__global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT>())) void qgemm_skinny_kernel(SkinnyParams p) {
+__global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm_skinny_kernel(SkinnyParams p) {
   static_assert(D == 1 || D == 2, "weights one or two steps ahead");
   static_assert(RT <= 4 && (!SW || RT >= 2), "tiles of a wavefront");
   constexpr bool KQ = is_kquant(QT);
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT>())) void qgemm_ski
   constexpr int XN = XR / 4;          // activation loads of a step
   constexpr int HT = SW ? RT / 2 : RT;  // tiles of one weight
   constexpr int TL = tile_lds<QT>();
-  constexpr int WLDS = wave_lds<QT, XR, RT>();
+  constexpr int WLDS = wave_lds<QT, XR, RT, KG>();
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int kg = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -357,7 +360,8 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT>())) void qgemm_ski
 
   // Accumulator tile (t, q): lane holds Y[m][n .. n+3] for m = m0 + 16q + lane % 16, n = n0 + 16t
   // + 4 (lane / 16) (SwiGLU: tiles 0 .. HT-1 gate, HT .. 2HT-1 up).  The KG partial tiles of an
-  // item meet in LDS (each wavefront's in its own part, between two barriers).
+  // item meet in LDS (each wavefront's in its own part, between two barriers); a lone wavefront
+  // has the sums in its registers.
   auto part = [&](int w, int u) { return *(const f32x4_t*)(lds + w * WLDS + (u * 64 + lane) * 16); };
   auto finish = [&](int item) {
     const int slab = slab_of(item), sub = item - slab * parts, m0 = sub * XR;
@@ -376,6 +380,14 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT>())) void qgemm_ski
       }
       if (m < M) store4(G.y, G.y_dtype, (size_t)m * N, nn, N, sum);
     };
+    if constexpr (KG == 1) {
+      sfor<HT * NB>([&](auto U_) {
+        constexpr int t = decltype(U_)::value / NB, q = decltype(U_)::value % NB;
+        put(t, q, tot[t][q], tot[SW ? HT + t : t][q]);
+      });
+      clear(tot);
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -469,7 +481,7 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT>())) void qgemm_ski
       finish(item);
       it = 0;
       if (++item >= item1) break;
-      __syncthreads();  // the partial tiles have been read
+      if constexpr (KG > 1) __syncthreads();  // the partial tiles have been read
     }
   }
 }
@@ -485,31 +497,38 @@ template <int QT, int XT, int XR, int RT, int KG, bool SW>
 const SkinnyKern& kern() {
   static std::atomic<int> residents[64];
   static const SkinnyKern k{(const void*)qgemm_skinny_kernel<QT, XT, XR, RT, RT == 4 ? 1 : 2, KG, SW>,
-                            KG * wave_lds<QT, XR, RT>(), 64 * KG, residents};
+                            KG * wave_lds<QT, XR, RT, KG>(), 64 * KG, residents};
   return k;
 }
 template <int QT, int XT, int XR>
-const SkinnyKern& kern_of(int rt, bool sw) {
+const SkinnyKern& kern_of(int rt, int kg, bool sw) {
+  if (kg == 1) {
+    if (sw) return rt == 4 ? kern<QT, XT, XR, 4, 1, true>() : kern<QT, XT, XR, 2, 1, true>();
+    return rt == 4   ? kern<QT, XT, XR, 4, 1, false>()
+           : rt == 2 ? kern<QT, XT, XR, 2, 1, false>()
+                     : kern<QT, XT, XR, 1, 1, false>();
+  }
   if (sw) return rt == 4 ? kern<QT, XT, XR, 4, 8, true>() : kern<QT, XT, XR, 2, 8, true>();
   return rt == 4   ? kern<QT, XT, XR, 4, 8, false>()
          : rt == 2 ? kern<QT, XT, XR, 2, 8, false>()
                    : kern<QT, XT, XR, 1, 8, false>();
 }
 template <int QT, int XT>
-const SkinnyKern& kern_of(int xr, int rt, bool sw) {
-  return xr == 8    ? kern_of<QT, XT, 8>(rt, sw)
-         : xr == 16 ? kern_of<QT, XT, 16>(rt, sw)
-                    : kern_of<QT, XT, 32>(rt, sw);
+const SkinnyKern& kern_of(int xr, int rt, int kg, bool sw) {
+  return xr == 8    ? kern_of<QT, XT, 8>(rt, kg, sw)
+         : xr == 16 ? kern_of<QT, XT, 16>(rt, kg, sw)
+                    : kern_of<QT, XT, 32>(rt, kg, sw);
 }
 
 // One translation unit per quant type instantiates the kernels (qgemm_skinny_<type>.hip).  xr: rows
-// of a block of M (8, 16, 32); rt: tiles per wavefront (1, 2, 4; SwiGLU 2, 4).
-const SkinnyKern& kern_q4k(bool f16, int xr, int rt, bool sw);
-const SkinnyKern& kern_q6k(bool f16, int xr, int rt, bool sw);
-const SkinnyKern& kern_q5k(bool f16, int xr, int rt, bool sw);
-const SkinnyKern& kern_q40(bool f16, int xr, int rt, bool sw);
-const SkinnyKern& kern_q41(bool f16, int xr, int rt, bool sw);
-const SkinnyKern& kern_q80(bool f16, int xr, int rt, bool sw);
+// of a block of M (8, 16, 32); rt: tiles per wavefront (1, 2, 4; SwiGLU 2, 4); kg: wavefronts (8, or
+// 1 for K <= 1024).
+const SkinnyKern& kern_q4k(bool f16, int xr, int rt, int kg, bool sw);
+const SkinnyKern& kern_q6k(bool f16, int xr, int rt, int kg, bool sw);
+const SkinnyKern& kern_q5k(bool f16, int xr, int rt, int kg, bool sw);
+const SkinnyKern& kern_q40(bool f16, int xr, int rt, int kg, bool sw);
+const SkinnyKern& kern_q41(bool f16, int xr, int rt, int kg, bool sw);
+const SkinnyKern& kern_q80(bool f16, int xr, int rt, int kg, bool sw);
 
 }  // namespace skinny
 }  // namespace mlxr

@@ -657,6 +657,51 @@ def test_skinny_tile_counts_match_oracle(cuda, qt, M, N, K):
     assert (d <= bound + 2.0**-24 * np.abs(ref)).all(), (d - bound).max()
 
 
+@pytest.mark.parametrize("qt,M,N,K", [(Q4K, 1, 17, 256), (Q6K, 8, 65, 512), (Q80, 9, 4100, 1024), (Q5K, 16, 33, 768),
+                                      (Q41, 17, 130, 32), (Q40, 33, 5000, 992), (Q4K, 40, 70000, 256), (Q6K, 100, 63, 1024)])
+def test_skinny_lone_wavefront_equals_eight(cuda, qt, M, N, K):
+    """K of up to 1024 (a super-block or less for each of eight wavefronts): one wavefront per workgroup
+    takes them in the order in which the eight are added, with the same bits for one, two and four
+    tiles, with a bias, as a grouped call and in the fused SwiGLU; the oracle within the bound of
+    test_skinny_tile_counts_match_oracle."""
+    import torch
+    w, pw = _packed(torch, qt, N, K, 811 + M, cuda)
+    _, pu = _packed(torch, qt, N, K, 812 + M, cuda)
+    x, xf = _act(torch, M, K, mx.BF16, 821 + M, cuda)
+    bias = torch.linspace(-1, 1, N, device=cuda)
+    got = {}
+    try:
+        mx.qgemm.test_force_skinny(True)
+        for tiles in (1, 2, 4):
+            for waves in (8, 1):
+                mx.qgemm.test_skinny_plan(tiles, waves)
+                got[tiles, waves] = [mx.q_gemm_dequant(x, pw, M, N, K, qt, out_dtype=torch.float32, path=mx.PATH_MFMA),
+                                     mx.q_gemm_dequant(x, pw, M, N, K, qt, bias=bias, path=mx.PATH_MFMA)]
+                if M > 4:
+                    got[tiles, waves] += mx.q_gemm_dequant_grouped(x, [pw, pu, pw], out_dtype=torch.float32, workspace=False)
+                    got[tiles, waves].append(mx.q_gemm_swiglu(x, pw, pu, out_dtype=torch.float32, workspace=False))
+    finally:
+        mx.qgemm.test_skinny_plan()
+        mx.qgemm.test_force_skinny(False)
+    torch.cuda.synchronize()
+    for k, ys in got.items():
+        for i, (y, y0) in enumerate(zip(ys, got[1, 8])):
+            assert torch.equal(y, y0), (k, i)
+    rows = slice(0, min(N, 600))
+    ref = orc.gemm_f64(int(qt), M, N, K, w, xf, w_to_bf16=True).astype(np.float64)[:, rows]
+    wabs = np.abs(orc.dequant(int(qt), N, K, w).reshape(N, K)[rows].astype(np.float64)) * (1 + 2.0**-8)
+    bound = np.abs(xf.astype(np.float64)) @ wabs.T * (32 + 8 + 1 + 8) * 2.0**-23
+    d = np.abs(got[4, 1][0].cpu().numpy().astype(np.float64)[:, rows] - ref)
+    assert (d <= bound + 2.0**-24 * np.abs(ref)).all(), (d - bound).max()
+
+
+def test_wide_weights_of_short_rows_take_lone_wavefronts(cuda):
+    """65536 x 1024 (Q4_K at M = 8 14.0 us with one wavefront per workgroup, 20.4 with eight) and 1536 x
+    1024 (5.7 and 4.1)."""
+    assert mx.qgemm.test_skinny_layout(Q4K, 65536, 1024, 8)[1] == 1
+    assert mx.qgemm.test_skinny_layout(Q4K, 1536, 1024, 8)[1] == 8
+
+
 @pytest.mark.parametrize("qt,M", [(Q4K, 8), (Q80, 5), (Q6K, 3)])
 def test_skinny_staged_f16_activations_match_oracle(cuda, qt, M):
     """fp16 activations (the fp16 MFMA, fp16-rounded weights) through the staged narrow
