@@ -127,10 +127,10 @@ int mlxr_qgemm_run_ex(int qtype, int N, int K, int group_size, const void* packe
                       void* y_dev, int y_dtype, int M, int path, void* stream);
 
 /* Device workspace bytes mlxr_qgemm_run_ws can use for an [M, N, K] problem; 0 when the
- * problem would not use one.  Tiled MFMA GEMMs (M > 32) whose workgroups would be too few to
- * fill the device split K over several workgroups and add the fp32 partials in a second
- * kernel; the workspace holds those partials (splits x M x N x 4 bytes).  The skinny kernel
- * leaves it untouched (a size is reported for some of its shapes too).  With the reported size,
+ * problem would not use one.  MFMA GEMMs whose workgroups would be too few to fill the device
+ * (tiled ones, M > 32, and skinny ones of few rows and a long K) split K over several workgroups
+ * and add the fp32 partials in a second kernel; the workspace holds those partials (splits x M x N
+ * x 4 bytes; a size is also reported for shapes that then run unsplit).  With the reported size,
  * calls with 32 < M <= 2048 run the skinny or the tiled kernel, whichever is estimated faster;
  * up to M = 256 mlxr_qgemm_run_ws ignores a smaller workspace (the call then runs as
  * mlxr_qgemm_run_ex: skinny kernel for M <= 64, tiled one above, unsplit).
@@ -185,9 +185,9 @@ typedef struct mlxr_qgemm_item {
 /* y_i[M, N_i] = X[M, K] . W_i[N_i, K]^T (+ bias_i) for `count` weights that read the same
  * activations -- the projections of one input, e.g. q/k/v or gate/up of a decoder layer.
  * Every item must have the same K.  Items of one quant type run up to four per launch
- * where the kernel allows it: the GEMV at M <= 4 (X staged once), the skinny MFMA kernel to
- * M = 64 and the tiled MFMA GEMM above (slabs or tile columns of the weights side by side); other
- * items run as mlxr_qgemm_run(..., MLXR_PATH_AUTO).  Results equal count separate mlxr_qgemm_run calls
+ * where the kernel allows it: the GEMV at M <= 4 (X staged once), the skinny or the tiled MFMA
+ * kernel (slabs or tile columns of the weights side by side; each weight on the kernel of its
+ * mlxr_qgemm_run call); other items run as mlxr_qgemm_run(..., MLXR_PATH_AUTO).  Results equal count separate mlxr_qgemm_run calls
  * bit for bit, with one exception at M <= 4: an item whose single call the automatic path
  * gives the skinny MFMA kernel (mlxr_qgemm_auto_path) stays in the GEMV launch unless its
  * weight is very large (N*K >= 128 Mi elements), and then equals its single call with
@@ -213,10 +213,12 @@ int mlxr_qgemm_grouped_workspace_size(int count, const mlxr_qgemm_item* items, i
 /* h[M, N] = swish(X . Wg^T) * (X . Wu^T): the gate/up half of a SwiGLU MLP
  * (reference core/graph/layers.cpp:391-414; swiglu_mlp_fused.metal:131-345 plans the
  * fusion).  gate_packed and up_packed are packed weights of the same type and [N, K].
- * At M <= 4 one launch computes both projections and the gating (no gate/up outputs ever
- * reach memory) and needs no workspace; above, it runs the two projections and
- * mlxr_swiglu, and the up projection goes to the caller's workspace of
- * mlxr_qgemm_swiglu_workspace_size bytes.  No counterpart in the reference's operator. */
+ * One launch computes both projections and the gating (no gate/up outputs ever reach memory): the
+ * GEMV at M <= 4, the skinny or the tiled MFMA kernel otherwise.  With a workspace of
+ * mlxr_qgemm_swiglu_workspace_size bytes, launches of too few workgroups split K and add one that
+ * reduces and gates; NULL or less runs unsplit.  Operands of 2 GiB or more run as the two
+ * projections and mlxr_swiglu, and then need the workspace for the up projection.  No counterpart
+ * in the reference's operator. */
 int mlxr_qgemm_swiglu_workspace_size(int qtype, int N, int K, int M, int h_dtype, size_t* bytes);
 int mlxr_qgemm_swiglu(int qtype, int N, int K, const void* gate_packed, const void* up_packed,
                       const void* x_dev, int x_dtype, void* h_dev, int h_dtype, int M,
@@ -277,7 +279,8 @@ int mlxr_qgemm_mlp_status(void* workspace_dev, void* stream);
  * mlxr_qgemm_test_skinny_stage: weight tiles a wavefront of
  * the skinny kernel takes: 0 one, 2 two, 3 and above four (SwiGLU: two, two, four), 1 restores
  * the choice by shape; mlxr_qgemm_test_skinny_plan sets them too (1, 2, 4), with the wavefronts of a
- * workgroup (8, or 1 where K <= 1024), each 0 by shape; tests use them to check every variant
+ * workgroup (8, or 1 where K <= 1024) and the splits of K over workgroups (where the call's
+ * workspace holds their partial sums), each 0 by shape; tests use them to check every variant
  * against the oracle.
  * All are process-wide (atomics).
  * mlxr_qgemm_test_kernels launches nothing: it tells which kernel would run each item, and which
@@ -295,7 +298,7 @@ int mlxr_qgemm_test_set_operand_limit(size_t bytes);
 int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks);
 int mlxr_qgemm_test_force_skinny(int on);
 int mlxr_qgemm_test_skinny_stage(int on);
-int mlxr_qgemm_test_skinny_plan(int tiles, int waves);
+int mlxr_qgemm_test_skinny_plan(int tiles, int waves, int splits);
 
 /* Deterministic synthetic inputs with the shapes/distributions of the benchmark
  * configurations (host memory).  Generator: SplitMix64 from `seed`; normals by

@@ -446,6 +446,10 @@ std::vector<Batch> call_batches(const std::vector<mlxr::RunArgs>& a, int M, bool
     for (int k = 0; k < bt.n; ++k) batch[k] = &a[(size_t)bt.idx[k]];
     if (batch_skinny(batch, bt.n, M, *ws ? ws_bytes : 0)) bt.kind = kGroupedSkinny;
   }
+  // a weight by itself may use the workspace
+  if (*ws && M <= kSkinnyOnlyMaxM)
+    for (Batch& bt : out)
+      if (bt.kind == kGroupedSkinny && bt.n == 1) bt.kind = kSingle;
   return out;
 }
 
@@ -781,14 +785,15 @@ int mlxr_qgemm_test_set_mlp_spin_limit(unsigned ticks) {
 }
 
 int mlxr_qgemm_test_skinny_stage(int on) {
-  return mlxr_qgemm_test_skinny_plan(on <= 0 ? 1 : on == 1 ? 0 : on == 2 ? 2 : 4, 0);
+  return mlxr_qgemm_test_skinny_plan(on <= 0 ? 1 : on == 1 ? 0 : on == 2 ? 2 : 4, 0, 0);
 }
 
-int mlxr_qgemm_test_skinny_plan(int tiles, int waves) {
-  if ((tiles != 0 && tiles != 1 && tiles != 2 && tiles != 4) || (waves != 0 && waves != 1 && waves != 8))
+int mlxr_qgemm_test_skinny_plan(int tiles, int waves, int splits) {
+  if ((tiles != 0 && tiles != 1 && tiles != 2 && tiles != 4) || (waves != 0 && waves != 1 && waves != 8) || splits < 0)
     return fail(MLXR_E_INVALID, "invalid skinny plan");
   mlxr::g_skinny_tiles.store(tiles, std::memory_order_relaxed);
   mlxr::g_skinny_waves.store(waves, std::memory_order_relaxed);
+  mlxr::g_skinny_splits.store(splits, std::memory_order_relaxed);
   return MLXR_OK;
 }
 

@@ -75,7 +75,7 @@ int device_cu_count();
 size_t device_lds_limit();
 
 // Skinny MFMA GEMM (qgemm_skinny.hip): any M in blocks of up to 32 rows, the weights streamed
-// once per block.  It takes no workspace.
+// once per block.  With a.ws, K of weights of few rows may be split over workgroups (M <= 32).
 hipError_t launch_skinny(const RunArgs& a, hipStream_t s);
 // Up to 4 weights of one quant type and K sharing x and M in one launch (skinny_group_fits);
 // equal to separate launches bit for bit.
@@ -85,8 +85,8 @@ double skinny_us(const RunArgs* const* items, int n, bool swiglu);
 // Its weight tiles per wavefront, wavefronts per workgroup and splits of K over workgroups.
 void skinny_layout(const RunArgs* const* items, int n, bool swiglu, int* layout);
 // What tests force on the skinny kernel, 0 by shape (default): weight tiles of a wavefront (1, 2, 4;
-// SwiGLU 2, 4), wavefronts of a workgroup (1, 8).
-extern std::atomic<int> g_skinny_tiles, g_skinny_waves;
+// SwiGLU 2, 4), wavefronts of a workgroup (1, 8), splits of K over workgroups.
+extern std::atomic<int> g_skinny_tiles, g_skinny_waves, g_skinny_splits;
 // Whether every operand of a is below operand_limit() and the launch's items are countable (else:
 // launch_mfma, which chunks); of a launch of n weights.
 bool skinny_fits(const RunArgs& a);

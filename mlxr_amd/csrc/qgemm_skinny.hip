@@ -10,20 +10,20 @@
 
 namespace mlxr {
 
-std::atomic<int> g_skinny_tiles{0}, g_skinny_waves{0};
+std::atomic<int> g_skinny_tiles{0}, g_skinny_waves{0}, g_skinny_splits{0};
 
 namespace {
 
 using namespace skinny;
 
-const SkinnyKern& kern_for(int qtype, bool f16, int xr, int rt, int kg, bool sw) {
+const SkinnyKern& kern_for(int qtype, bool f16, int xr, int rt, int kg, bool sw, bool split) {
   switch (qtype) {
-    case QT_Q4_K: return kern_q4k(f16, xr, rt, kg, sw);
-    case QT_Q6_K: return kern_q6k(f16, xr, rt, kg, sw);
-    case QT_Q5_K: return kern_q5k(f16, xr, rt, kg, sw);
-    case QT_Q4_0: return kern_q40(f16, xr, rt, kg, sw);
-    case QT_Q4_1: return kern_q41(f16, xr, rt, kg, sw);
-    default: return kern_q80(f16, xr, rt, kg, sw);
+    case QT_Q4_K: return kern_q4k(f16, xr, rt, kg, sw, split);
+    case QT_Q6_K: return kern_q6k(f16, xr, rt, kg, sw, split);
+    case QT_Q5_K: return kern_q5k(f16, xr, rt, kg, sw, split);
+    case QT_Q4_0: return kern_q40(f16, xr, rt, kg, sw, split);
+    case QT_Q4_1: return kern_q41(f16, xr, rt, kg, sw, split);
+    default: return kern_q80(f16, xr, rt, kg, sw, split);
   }
 }
 
@@ -47,9 +47,9 @@ int residents(const SkinnyKern& k, hipError_t* e) {
 }
 
 // How a launch is laid out: weight tiles of a wavefront, wavefronts of a workgroup (8, or 1 for short
-// K), and its estimated time.
+// K), splits of K over workgroups, and its estimated time.
 struct Plan {
-  int rt, kg;
+  int rt, kg, ks;
   double us;
 };
 
@@ -106,30 +106,47 @@ double plan_us(int qtype, int xr, int rt, int kg, long items, long turns, int oc
 // order, and the sums are the same bits: a wide weight then need not meet in LDS once per item
 // (Q4_K 65536 x 1024 at M = 8 20.4 -> 14.0 us, 16384 x 256 7.5 -> 4.2; 1536 x 1024 4.1 with eight
 // wavefronts, 5.7 with one).
+// With a workspace, a long K of a weight of few rows is split over workgroups too, which a second
+// launch adds (Q4_K 1024 x 14336 at M = 16 12.4 -> 8.7 us; Q8_0 2048 x 14336 18.0 -> 15.3; 4096 x
+// 14336 20.9, split 25.2).  Fewer than four turns pay for it at M = 17 .. 32 and in SwiGLU (Q8_0 896 x
+// 4864 at M = 32 11.1 -> 8.8 us); elsewhere they gain 8% at most and stay whole.
 Plan plan_for(const RunArgs* const* items, int n, bool swiglu) {
   const RunArgs& a = *items[0];
   const int M = a.M, K = a.L.K, xr = rows_of_block(M);
   const bool f16 = a.x_dtype == DT_F16;
-  const int tiles = g_skinny_tiles.load(std::memory_order_relaxed), waves = g_skinny_waves.load(std::memory_order_relaxed);
+  const int tiles = g_skinny_tiles.load(std::memory_order_relaxed), waves = g_skinny_waves.load(std::memory_order_relaxed),
+            splits = g_skinny_splits.load(std::memory_order_relaxed);
   const int nsb = (K + 255) / 256, turns = (nsb + 7) / 8;
   double bytes = 0;
   for (int i = 0; i < n; ++i) bytes += (double)items[i]->L.total;
-  Plan best{0, 0, 1e30};
-  auto consider = [&](int rt, int kg) {
+  Plan best{0, 0, 0, 1e30};
+  auto consider = [&](int rt, int kg, int ks) {
     const int rows = (swiglu ? 8 : 16) * rt;
     long slabs = 0;
     for (int i = 0; i < (swiglu ? 1 : n); ++i) slabs += (items[i]->L.N + rows - 1) / rows;
     hipError_t e;
-    const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, kg, swiglu), &e));
-    const int mblocks = (M + xr - 1) / xr;
-    const double us = plan_us(a.L.qtype, xr, rt, kg, slabs * mblocks, kg == 1 ? nsb : turns, occ, mblocks, bytes);
-    if (us < best.us) best = Plan{rt, kg, us};
+    const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, kg, swiglu, ks > 1), &e));
+    const long parts = (long)((M + xr - 1) / xr) * ks, nitems = slabs * parts;
+    if (ks > 1 && (uint64_t)(nitems * parts) >= (1ull << 32)) return;
+    double us = plan_us(a.L.qtype, xr, rt, kg, nitems, kg == 1 ? nsb : (turns + ks - 1) / ks, occ,
+                        (M + xr - 1) / xr, bytes);
+    if (ks > 1) us += 3.1 + (double)ks * M * a.L.N * (swiglu ? 16 : 8) / 6.3e6;  // the second launch
+    if (us < best.us) best = Plan{rt, kg, ks, us};
   };
   for (int rt : {1, 2, 4}) {
     if (swiglu && rt == 1) continue;
     if (tiles && rt != (swiglu ? std::max(tiles, 2) : tiles)) continue;
-    if (waves != 1 || K > 1024) consider(rt, 8);
-    if (waves != 8 && K <= 1024) consider(rt, 1);
+    if (waves != 1 || K > 1024) consider(rt, 8, 1);
+    if (waves != 8 && K <= 1024) consider(rt, 1, 1);
+  }
+  if ((n == 1 || swiglu) && a.ws && tiles == 0 && waves == 0 && (turns >= 4 || (M <= 32 && (M > 16 || swiglu)) || splits > 1)) {
+    const size_t plane = (size_t)M * (size_t)a.L.N * (swiglu ? 8u : 4u);
+    if (splits > 1) best.us = 1e30;
+    for (int s = 2; s <= std::min(turns, 16); ++s) {
+      const int tps = (turns + s - 1) / s, ks = (turns + tps - 1) / tps;
+      if (ks == s && (splits == 0 || splits == s) && ks * plane <= a.ws_bytes) consider(swiglu ? 2 : 1, 8, ks);
+    }
+    if (best.us == 1e30) consider(swiglu ? 2 : 1, 8, 1);
   }
   return best;
 }
@@ -138,7 +155,7 @@ hipError_t launch_any(const RunArgs* const* items, int n, bool swiglu, hipStream
   SkinnyParams sp;
   const RunArgs& a = *items[0];
   const Plan pl = plan_for(items, n, swiglu);
-  const int xr = rows_of_block(a.M), rows = (swiglu ? 8 : 16) * pl.rt;
+  const int xr = rows_of_block(a.M), rows = (swiglu ? 8 : 16) * pl.rt, turns = (a.L.K + 256 * pl.kg - 1) / (256 * pl.kg);
   int slabs = 0;
   for (int i = 0; i < MAX_SG; ++i) {
     const RunArgs& b = *items[i < n ? i : 0];
@@ -157,9 +174,15 @@ hipError_t launch_any(const RunArgs* const* items, int n, bool swiglu, hipStream
   sp.M = a.M;
   sp.K = a.L.K;
   sp.ngroups = n;
-  sp.parts = (a.M + xr - 1) / xr;
+  sp.parts = (a.M + xr - 1) / xr * pl.ks;
+  sp.ks = pl.ks;
+  sp.kdiv = pl.ks > 1 ? (uint32_t)(((1ull << 32) + pl.ks - 1) / pl.ks) : 0u;
   sp.mdiv = sp.parts > 1 ? (uint32_t)(((1ull << 32) + sp.parts - 1) / sp.parts) : 0u;
-  const SkinnyKern& k = kern_for(a.L.qtype, a.x_dtype == DT_F16, xr, pl.rt, pl.kg, swiglu);
+  sp.tps = (turns + pl.ks - 1) / pl.ks;
+  sp.ws = pl.ks > 1 ? (float*)a.ws : nullptr;
+  sp.ws_ld = (swiglu ? 2 : 1) * a.L.N;
+  sp.ws_split = (size_t)a.M * (size_t)sp.ws_ld;
+  const SkinnyKern& k = kern_for(a.L.qtype, a.x_dtype == DT_F16, xr, pl.rt, pl.kg, swiglu, pl.ks > 1);
   hipError_t e = hipSuccess;
   const int occ = residents(k, &e);
   if (occ == 0) return e;
@@ -167,12 +190,17 @@ hipError_t launch_any(const RunArgs* const* items, int n, bool swiglu, hipStream
   sp.per = nitems / grid;
   sp.rem = nitems % grid;
   void* args[1] = {&sp};
-  return hipLaunchKernel(k.fn, dim3((unsigned)grid), dim3((unsigned)k.threads), args, (size_t)k.lds, s);
+  e = hipLaunchKernel(k.fn, dim3((unsigned)grid), dim3((unsigned)k.threads), args, (size_t)k.lds, s);
+  if (e != hipSuccess || pl.ks == 1) return e;
+  const RunArgs& u = *items[n - 1];
+  return swiglu ? launch_splitk_reduce_swiglu(sp.ws, sp.ws_split, pl.ks, a.bias, u.bias, a.bias_dtype, a.y, a.y_dtype,
+                                              a.M, a.L.N, s)
+                : launch_splitk_reduce(sp.ws, sp.ws_split, pl.ks, a.bias, a.bias_dtype, a.y, a.y_dtype, a.M, a.L.N, s);
 }
 
 // Splits of K that the workspace sizes reported for these calls hold (skinny_workspace_bytes).  The
 // sizes stay what callers have been told, as they decide which calls mlxr_qgemm_run_noalloc
-// takes; the kernel splits K inside a workgroup and leaves the workspace untouched.
+// takes; a launch uses as many of the splits as pay, or none.
 int splits_of(int groups, int nkt, int steps) {  // at most `groups`, of whole `steps` of the nkt
   const int ks = std::max(1, std::min(groups, nkt / steps));
   const int per = ((nkt + ks - 1) / ks + steps - 1) / steps * steps;
@@ -211,7 +239,7 @@ void skinny_layout(const RunArgs* const* items, int n, bool swiglu, int* layout)
   const Plan pl = plan_for(items, n, swiglu);
   layout[0] = pl.rt;
   layout[1] = pl.kg;
-  layout[2] = 1;
+  layout[2] = pl.ks;
 }
 
 size_t skinny_swiglu_workspace_bytes(int M, int N, int K) {

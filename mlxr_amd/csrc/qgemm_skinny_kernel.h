@@ -14,7 +14,9 @@
 // tiles of the KG wavefronts meet in LDS at the end and are added in wavefront order.  KG is 8; a
 // lone wavefront (KG = 1, K <= 1024, where the eight have a super-block or less) adds the same
 // super-blocks in the same order and has neither barrier nor exchange.  So an output's sum does not
-// depend on how many rows or weights a launch holds.
+// depend on how many rows or weights a launch holds, unless K is split over workgroups (SPLIT):
+// then each item has some turns (KG super-blocks) of K, and a second launch adds their fp32 partial
+// sums.
 //
 // The activations go through LDS, read with whole 256-byte row segments.  (Read straight
 // into the operand layout, one load instruction touches 64 different 64-byte segments and
@@ -53,9 +55,14 @@ struct SkinnyGroup {
 struct SkinnyParams {
   const void* x;
   int M, K;
-  int parts;      // items of a slab: blocks of XR rows of M
+  int parts;      // items of a slab: blocks of XR rows of M, times splits of K
   uint32_t mdiv;  // ceil(2^32 / parts): item / parts by a multiplication (parts > 1)
   int per, rem;   // items of a workgroup; the first rem workgroups have one more
+  int ks, tps;    // split: splits of K, turns (KG super-blocks) of K of an item
+  uint32_t kdiv;  // ceil(2^32 / ks)
+  float* ws;      // split: fp32 partials, split s at ws + s * ws_split, rows of ws_ld (SwiGLU: gate, up)
+  size_t ws_split;
+  int ws_ld;
   int ngroups;
   // SwiGLU: g[0] gate, g[1] up; half of a wavefront's tiles are rows of gate, half the same rows of up
   SkinnyGroup g[MAX_SG];
@@ -199,14 +206,15 @@ constexpr int wave_lds() {
 
 // Wavefronts per SIMD the registers are bounded for: 4 (two workgroups on a CU) where that takes
 // no more than a handful of spills, else 2 (lone wavefronts: 3).
-template <int QT, int XR, int RT, int KG>
+template <int QT, int XR, int RT, int KG, bool SPLIT>
 constexpr int skinny_occ() {
+  if (SPLIT) return 2;  // no more than a workgroup per CU
   if (KG == 1 && RT == 4 && XR <= 16) return 3;
   return XR > 16 || QT == QT_Q6_K || QT == QT_Q8_0 || (QT == QT_Q5_K && XR == 16 && RT == 4) ? 2 : 4;
 }
 
-template <int QT, int XT, int XR, int RT, int D, int KG, bool SW>
-__global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm_skinny_kernel(SkinnyParams p) {
+template <int QT, int XT, int XR, int RT, int D, int KG, bool SW, bool SPLIT>
+__global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG, SPLIT>())) void qgemm_skinny_kernel(SkinnyParams p) {
   static_assert(D == 1 || D == 2, "weights one or two steps ahead");
   static_assert(RT <= 4 && (!SW || RT >= 2), "tiles of a wavefront");
   constexpr bool KQ = is_kquant(QT);
@@ -226,7 +234,7 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
   const int item0 = f * p.per + min(f, p.rem), item1 = item0 + p.per + (f < p.rem ? 1 : 0);
   const int r = lane & 15, j = lane >> 4;
   auto slab_of = [&](int item) { return parts == 1 ? item : (int)__umulhi((uint32_t)item, p.mdiv); };
-  const int nit = 2 * ((((K + 255) >> 8) + KG - 1) / KG);  // steps per item, even
+  const int nit = SPLIT ? 2 * p.tps : 2 * ((((K + 255) >> 8) + KG - 1) / KG);  // steps per item, even
 
   // LDS of this wavefront: activations, two tile slots, headers
   uint8_t* const xl = lds + kg * WLDS;
@@ -241,10 +249,14 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
   uint32_t xrow[XN];
   u32x4_t xs[XN];
   int x_part = 0, x_it = 0;  // next step whose activations are loaded
+  auto block_of = [&](int part) { return SPLIT ? (int)__umulhi((uint32_t)part, p.kdiv) : part; };  // of M
+  auto split_of = [&](int part) { return part - block_of(part) * p.ks; };
   auto open_x = [&](int part) {
     x_part = part;
+    x_it = SPLIT ? split_of(part) * nit : 0;
+    const int m0 = block_of(part) * XR;
 #pragma unroll
-    for (int q = 0; q < XN; ++q) xrow[q] = (uint32_t)(min(part * XR + 4 * q + j, M - 1) * K + 8 * r) * 2u;
+    for (int q = 0; q < XN; ++q) xrow[q] = (uint32_t)(min(m0 + 4 * q + j, M - 1) * K + 8 * r) * 2u;
   };
   auto issue_x = [&]() {
     const uint32_t k0 = (uint32_t)(256 * (KG * (x_it >> 1) + kg) + 128 * (x_it & 1));
@@ -252,7 +264,7 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
     const uint32_t so = k0 < (uint32_t)K ? k0 * 2u : 0u;  // scalar offsets stay inside the buffer
 #pragma unroll
     for (int q = 0; q < XN; ++q) xs[q] = __builtin_amdgcn_raw_buffer_load_b128(RX, in ? xrow[q] : OOB, so, 0);
-    if (++x_it == nit) {
+    if (++x_it == (SPLIT ? (split_of(x_part) + 1) * nit : nit)) {
       x_it = 0;
       if (parts > 1) open_x(x_part + 1 == parts ? 0 : x_part + 1);
     }
@@ -289,8 +301,13 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
     }
     return gi;
   };
+  int w_item = item0, w_it = 0, w_end = nit;  // next step whose weights are loaded
   auto open_w = [&](int item) {
     const int slab = slab_of(item);
+    if constexpr (SPLIT) {
+      w_it = split_of(item - slab * parts) * nit;
+      w_end = w_it + nit;
+    }
     const SkinnyGroup& G = p.g[group_of(slab)];
     wN = G.N;
     wn0 = (slab - G.slab0) * 16 * HT;
@@ -300,7 +317,6 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
   const int lr = lane >> 2, lp = (lane & 3) ^ (lane >> 4);  // row and piece this lane loads
   const int slot = 4 * r + (j ^ (r >> 2));                  // where operand (r, j) is found
   const uint32_t vs = (uint32_t)lr * (uint32_t)nsub + 8u * kg + lp;
-  int w_item = item0, w_it = 0;  // next step whose weights are loaded
   Raw<QT> raw[D][RT];
   Hdr<QT> hdr[SW ? 2 : 1];  // lane 16 t + row: tile t's super-block header of that row
   // tile t of step it of an item, this wavefront: half it % 2 of super-block KG * (it / 2) + kg
@@ -338,8 +354,8 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
   auto next_w = [&](auto HALF) {
     ++w_it;
     if constexpr (decltype(HALF)::value == 1) {
-      if (w_it == nit) {
-        w_it = 0;
+      if (w_it == (SPLIT ? w_end : nit)) {
+        if constexpr (!SPLIT) w_it = 0;
         if (++w_item < item1) open_w(w_item);
       }
     }
@@ -364,12 +380,20 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG>())) void qgemm
   // has the sums in its registers.
   auto part = [&](int w, int u) { return *(const f32x4_t*)(lds + w * WLDS + (u * 64 + lane) * 16); };
   auto finish = [&](int item) {
-    const int slab = slab_of(item), sub = item - slab * parts, m0 = sub * XR;
+    const int slab = slab_of(item), sub = item - slab * parts, m0 = block_of(sub) * XR;
     const SkinnyGroup& G = p.g[group_of(slab)];
     const int N = G.N, n0 = (slab - G.slab0) * 16 * HT;
     // sums of tile t, block q of X (and of up's)
     auto put = [&](int t, int q, f32x4_t sum, const f32x4_t& up) {
       const int m = m0 + q * 16 + r, nn = n0 + 16 * t + 4 * j;
+      if constexpr (SPLIT) {  // this split's partial sums, no bias
+        float* const w = p.ws + (size_t)split_of(sub) * p.ws_split + (size_t)m * p.ws_ld;
+        if (m < M) {
+          store4(w, DT_F32, 0, nn, N, sum);
+          if constexpr (SW) store4(w + N, DT_F32, 0, nn, N, up);
+        }
+        return;
+      }
       if constexpr (SW) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] = swiglu1(sum[e], up[e]);
@@ -493,42 +517,43 @@ struct SkinnyKern {
   std::atomic<int>* residents;
 };
 
-template <int QT, int XT, int XR, int RT, int KG, bool SW>
+template <int QT, int XT, int XR, int RT, int KG, bool SW, bool SPLIT>
 const SkinnyKern& kern() {
   static std::atomic<int> residents[64];
-  static const SkinnyKern k{(const void*)qgemm_skinny_kernel<QT, XT, XR, RT, RT == 4 ? 1 : 2, KG, SW>,
+  static const SkinnyKern k{(const void*)qgemm_skinny_kernel<QT, XT, XR, RT, RT == 4 ? 1 : 2, KG, SW, SPLIT>,
                             KG * wave_lds<QT, XR, RT, KG>(), 64 * KG, residents};
   return k;
 }
 template <int QT, int XT, int XR>
-const SkinnyKern& kern_of(int rt, int kg, bool sw) {
+const SkinnyKern& kern_of(int rt, int kg, bool sw, bool split) {
+  if (split) return sw ? kern<QT, XT, XR, 2, 8, true, true>() : kern<QT, XT, XR, 1, 8, false, true>();
   if (kg == 1) {
-    if (sw) return rt == 4 ? kern<QT, XT, XR, 4, 1, true>() : kern<QT, XT, XR, 2, 1, true>();
-    return rt == 4   ? kern<QT, XT, XR, 4, 1, false>()
-           : rt == 2 ? kern<QT, XT, XR, 2, 1, false>()
-                     : kern<QT, XT, XR, 1, 1, false>();
+    if (sw) return rt == 4 ? kern<QT, XT, XR, 4, 1, true, false>() : kern<QT, XT, XR, 2, 1, true, false>();
+    return rt == 4   ? kern<QT, XT, XR, 4, 1, false, false>()
+           : rt == 2 ? kern<QT, XT, XR, 2, 1, false, false>()
+                     : kern<QT, XT, XR, 1, 1, false, false>();
   }
-  if (sw) return rt == 4 ? kern<QT, XT, XR, 4, 8, true>() : kern<QT, XT, XR, 2, 8, true>();
-  return rt == 4   ? kern<QT, XT, XR, 4, 8, false>()
-         : rt == 2 ? kern<QT, XT, XR, 2, 8, false>()
-                   : kern<QT, XT, XR, 1, 8, false>();
+  if (sw) return rt == 4 ? kern<QT, XT, XR, 4, 8, true, false>() : kern<QT, XT, XR, 2, 8, true, false>();
+  return rt == 4   ? kern<QT, XT, XR, 4, 8, false, false>()
+         : rt == 2 ? kern<QT, XT, XR, 2, 8, false, false>()
+                   : kern<QT, XT, XR, 1, 8, false, false>();
 }
 template <int QT, int XT>
-const SkinnyKern& kern_of(int xr, int rt, int kg, bool sw) {
-  return xr == 8    ? kern_of<QT, XT, 8>(rt, kg, sw)
-         : xr == 16 ? kern_of<QT, XT, 16>(rt, kg, sw)
-                    : kern_of<QT, XT, 32>(rt, kg, sw);
+const SkinnyKern& kern_of(int xr, int rt, int kg, bool sw, bool split) {
+  return xr == 8    ? kern_of<QT, XT, 8>(rt, kg, sw, split)
+         : xr == 16 ? kern_of<QT, XT, 16>(rt, kg, sw, split)
+                    : kern_of<QT, XT, 32>(rt, kg, sw, split);
 }
 
 // One translation unit per quant type instantiates the kernels (qgemm_skinny_<type>.hip).  xr: rows
 // of a block of M (8, 16, 32); rt: tiles per wavefront (1, 2, 4; SwiGLU 2, 4); kg: wavefronts (8, or
-// 1 for K <= 1024).
-const SkinnyKern& kern_q4k(bool f16, int xr, int rt, int kg, bool sw);
-const SkinnyKern& kern_q6k(bool f16, int xr, int rt, int kg, bool sw);
-const SkinnyKern& kern_q5k(bool f16, int xr, int rt, int kg, bool sw);
-const SkinnyKern& kern_q40(bool f16, int xr, int rt, int kg, bool sw);
-const SkinnyKern& kern_q41(bool f16, int xr, int rt, int kg, bool sw);
-const SkinnyKern& kern_q80(bool f16, int xr, int rt, int kg, bool sw);
+// 1 for K <= 2048); split: K split over workgroups (kg = 8 and the fewest tiles).
+const SkinnyKern& kern_q4k(bool f16, int xr, int rt, int kg, bool sw, bool split);
+const SkinnyKern& kern_q6k(bool f16, int xr, int rt, int kg, bool sw, bool split);
+const SkinnyKern& kern_q5k(bool f16, int xr, int rt, int kg, bool sw, bool split);
+const SkinnyKern& kern_q40(bool f16, int xr, int rt, int kg, bool sw, bool split);
+const SkinnyKern& kern_q41(bool f16, int xr, int rt, int kg, bool sw, bool split);
+const SkinnyKern& kern_q80(bool f16, int xr, int rt, int kg, bool sw, bool split);
 
 }  // namespace skinny
 }  // namespace mlxr

@@ -5,8 +5,8 @@
 namespace mlxr {
 namespace skinny {
 
-const SkinnyKern& kern_q5k(bool f16, int xr, int rt, int kg, bool sw) {
-  return f16 ? kern_of<QT_Q5_K, X_F16>(xr, rt, kg, sw) : kern_of<QT_Q5_K, X_BF16>(xr, rt, kg, sw);
+const SkinnyKern& kern_q5k(bool f16, int xr, int rt, int kg, bool sw, bool split) {
+  return f16 ? kern_of<QT_Q5_K, X_F16>(xr, rt, kg, sw, split) : kern_of<QT_Q5_K, X_BF16>(xr, rt, kg, sw, split);
 }
 
 }  // namespace skinny

@@ -90,7 +90,7 @@ _SIGS = {
     "mlxr_qgemm_test_force_tiled": (ctypes.c_int, [ctypes.c_int]),
     "mlxr_qgemm_test_kernels": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_void_p]),
     "mlxr_qgemm_test_skinny_layout": (ctypes.c_int, [ctypes.c_int] * 5 + [ctypes.c_size_t, ctypes.c_void_p]),
-    "mlxr_qgemm_test_skinny_plan": (ctypes.c_int, [ctypes.c_int] * 2),
+    "mlxr_qgemm_test_skinny_plan": (ctypes.c_int, [ctypes.c_int] * 3),
     "mlxr_qgemm_test_skinny_stage": (ctypes.c_int, [ctypes.c_int]),
     "mlxr_qgemm_auto_path": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                              ctypes.POINTER(ctypes.c_int)]),
@@ -475,10 +475,11 @@ def test_skinny_stage(mode):
     _check(lib().mlxr_qgemm_test_skinny_stage(int(mode)))
 
 
-def test_skinny_plan(tiles=0, waves=0):
+def test_skinny_plan(tiles=0, waves=0, splits=0):
     """Test hook, 0 by shape: weight tiles a wavefront of the skinny kernel takes (1, 2, 4; SwiGLU 2,
-    4), wavefronts of a workgroup (8, or 1 where K <= 1024)."""
-    _check(lib().mlxr_qgemm_test_skinny_plan(int(tiles), int(waves)))
+    4), wavefronts of a workgroup (8, or 1 where K <= 1024), splits of K over workgroups (where
+    the call's workspace holds their partial sums)."""
+    _check(lib().mlxr_qgemm_test_skinny_plan(int(tiles), int(waves), int(splits)))
 
 
 def test_skinny_layout(qtype, N, K, M, swiglu=False, workspace_bytes=0):

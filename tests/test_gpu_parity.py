@@ -702,6 +702,102 @@ def test_wide_weights_of_short_rows_take_lone_wavefronts(cuda):
     assert mx.qgemm.test_skinny_layout(Q4K, 1536, 1024, 8)[1] == 8
 
 
+@pytest.mark.parametrize("qt,M,N,K,ydt,splits", [(Q4K, 5, 100, 4352, "f32", 3), (Q6K, 16, 1024, 8192, "f32", 4),
+                                                 (Q80, 17, 63, 6176, "f16", 2), (Q5K, 32, 130, 4096, "bf16", 2),
+                                                 (Q41, 33, 66, 8224, "f32", 5), (Q40, 64, 257, 14336, "f32", 7),
+                                                 (Q4K, 70, 48, 10240, "bf16", 5), (Q6K, 64, 3000, 10240, "f32", 5)])
+def test_skinny_split_k_over_workgroups(cuda, qt, M, N, K, ydt, splits):
+    """K split over workgroups (partial sums in the workspace, added by a second launch): the oracle
+    within the bound of test_skinny_tile_counts_match_oracle with an addition per split, with a
+    bias, for every output type and ragged N, M in several blocks, a last split that is shorter or ends
+    inside a turn; the same bits on repeat; nothing written past the partial sums.  A workspace
+    that does not hold them gives the unsplit result."""
+    import torch
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[ydt]
+    code = {"bf16": mx.BF16, "f16": mx.F16, "f32": mx.F32}[ydt]
+    w, pw = _packed(torch, qt, N, K, 911 + M, cuda)
+    x, xf = _act(torch, M, K, mx.BF16, 921 + M, cuda)
+    bias = torch.linspace(-1, 1, N, device=cuda)
+    need = splits * M * N * 4
+    L, s = mx.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def run(nbytes):
+        y = torch.full((M, N), float("nan"), dtype=tdt, device=cuda)
+        ws = torch.full((need // 4 + 64,), 7.5, device=cuda)
+        rc = L.mlxr_qgemm_run_ws(int(qt), N, K, 0, pw.data_ptr(), x.data_ptr(), mx.BF16, bias.data_ptr(), mx.F32,
+                                 y.data_ptr(), code, M, mx.PATH_MFMA, ws.data_ptr(), nbytes, s)
+        assert rc == 0, L.mlxr_qgemm_last_error()
+        torch.cuda.synchronize()
+        return y, ws
+
+    try:
+        mx.qgemm.test_force_skinny(True)
+        whole, ws = run(0)
+        assert (ws == 7.5).all()
+        mx.qgemm.test_skinny_plan(0, 0, splits)
+        assert mx.qgemm.test_skinny_layout(qt, N, K, M, False, need)[2] == splits
+        y, ws = run(need)
+        assert (ws[need // 4:] == 7.5).all() and (ws[:need // 4] != 7.5).any()
+        assert torch.equal(run(need)[0], y)
+        short, ws = run(need - 1)
+        assert (ws == 7.5).all() and torch.equal(short, whole)
+    finally:
+        mx.qgemm.test_skinny_plan()
+        mx.qgemm.test_force_skinny(False)
+    ref = orc.gemm_f64(int(qt), M, N, K, w, xf, bias=bias.cpu().numpy(), w_to_bf16=True).astype(np.float64)
+    wabs = np.abs(orc.dequant(int(qt), N, K, w).reshape(N, K).astype(np.float64)) * (1 + 2.0**-8)
+    bound = (np.abs(xf.astype(np.float64)) @ wabs.T + 1) * (32 + 8 + K // 2048 + 1 + 8 + splits + 1) * 2.0**-23
+    out = {"f32": 2.0**-24, "f16": 2.0**-11, "bf16": 2.0**-8}[ydt]
+    for v in (y, whole):
+        d = np.abs(v.double().cpu().numpy() - ref)
+        assert (d <= bound * (1 + out) + out * np.abs(ref) + (2.0**-24 if ydt == "f16" else 0)).all(), (d - bound).max()
+
+
+@pytest.mark.parametrize("qt,M,N,K,splits", [(Q4K, 8, 100, 8192, 4), (Q6K, 24, 33, 4352, 3), (Q80, 40, 130, 4128, 3)])
+def test_skinny_split_k_swiglu(cuda, qt, M, N, K, splits):
+    """The fused SwiGLU split over workgroups equals the whole one within its sums' error: gate and up
+    within the bound of the split, the gating's own error as in
+    test_swiglu_of_narrow_weights_takes_skinny_kernel."""
+    import torch
+    (wg, pg), (wu, pu) = _packed(torch, qt, N, K, 931, cuda), _packed(torch, qt, N, K, 932, cuda)
+    x, xf = _act(torch, M, K, mx.BF16, 933 + M, cuda)
+    L, s = mx.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    need = ctypes.c_size_t(0)
+    assert L.mlxr_qgemm_swiglu_workspace_size(int(qt), N, K, M, mx.F32, ctypes.byref(need)) == 0
+    assert need.value >= splits * M * N * 8, need.value
+    h = torch.full((M, N), float("nan"), device=cuda)
+    ws = torch.full((need.value // 4,), 7.5, device=cuda)
+    try:
+        mx.qgemm.test_force_skinny(True)
+        mx.qgemm.test_skinny_plan(0, 0, splits)
+        rc = L.mlxr_qgemm_swiglu(int(qt), N, K, pg.data_ptr(), pu.data_ptr(), x.data_ptr(), mx.BF16, h.data_ptr(), mx.F32,
+                                 M, ws.data_ptr(), need.value, s)
+        assert rc == 0, L.mlxr_qgemm_last_error()
+        torch.cuda.synchronize()
+    finally:
+        mx.qgemm.test_skinny_plan()
+        mx.qgemm.test_force_skinny(False)
+    assert (ws[:splits * M * N * 2] != 7.5).any()
+    g, u = (orc.gemm_f64(int(qt), M, N, K, w, xf, w_to_bf16=True).astype(np.float64) for w in (wg, wu))
+    eg, eu = (np.abs(xf.astype(np.float64)) @ (np.abs(orc.dequant(int(qt), N, K, w).reshape(N, K).astype(np.float64)) *
+                                               (1 + 2.0**-8)).T * (32 + 8 + K // 2048 + 1 + 8 + splits) * 2.0**-23
+              for w in (wg, wu))
+    sw = g / (1 + np.exp(-g))
+    ref = sw * u
+    # |d swish| <= 1.1 |d g|
+    bound = 1.1 * eg * (np.abs(u) + eu) + np.abs(sw) * eu + (16 + 2 * np.abs(g)) * 2.0**-23 * np.abs(ref) + 2.0**-126 * (1 + np.abs(u))
+    assert (np.abs(h.double().cpu().numpy() - ref) <= bound).all()
+
+
+def test_few_rows_of_long_k_are_split(cuda):
+    """1024 x 14336 at M = 16 (Q4_K 8.7 us split, 12.4 whole), with the workspace asked for; 4096 x 14336
+    stays whole (20.9 us, split 25.2)."""
+    for N, split in ((1024, True), (4096, False)):
+        need = mx.workspace_size(Q4K, N, 14336, 16)
+        assert need > 0 and (mx.qgemm.test_skinny_layout(Q4K, N, 14336, 16, False, need)[2] > 1) == split
+        assert mx.qgemm.test_skinny_layout(Q4K, N, 14336, 16)[2] == 1
+
+
 @pytest.mark.parametrize("qt,M", [(Q4K, 8), (Q80, 5), (Q6K, 3)])
 def test_skinny_staged_f16_activations_match_oracle(cuda, qt, M):
     """fp16 activations (the fp16 MFMA, fp16-rounded weights) through the staged narrow
