@@ -105,12 +105,12 @@ __device__ __forceinline__ void decode_hdr1(const Hdr<QT>& h, uint32_t sel, Scal
   }
 }
 
-// Four consecutive outputs of one row.
+// Four consecutive outputs of one row, in one store where y's address and rows are aligned to it.
 __device__ __forceinline__ void store4(void* y, int y_dtype, size_t rowbase, int nn, int N, const f32x4_t& v) {
   const uint2 h = y_dtype == DT_BF16 ? make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]))
                                      : make_uint2(pack2<X_F16>(v[0], v[1]), pack2<X_F16>(v[2], v[3]));
   const size_t at = rowbase + nn;
-  if ((N & 3) == 0 && nn + 3 < N) {
+  if ((N & 3) == 0 && ((uintptr_t)y & (y_dtype == DT_F32 ? 15 : 7)) == 0 && nn + 3 < N) {
     if (y_dtype == DT_F32) *(f32x4_t*)((float*)y + at) = v;
     else *(uint2*)((uint16_t*)y + at) = h;
   } else {

@@ -798,6 +798,35 @@ def test_few_rows_of_long_k_are_split(cuda):
         assert mx.qgemm.test_skinny_layout(Q4K, N, 14336, 16)[2] == 1
 
 
+@pytest.mark.parametrize("ydt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("M,K", [(8, 2048), (24, 256), (40, 2048)])
+def test_skinny_outputs_at_any_element_address(cuda, ydt, M, K):
+    """Outputs that start at any element of a buffer (the skinny kernel stores four at a time only where
+    their address is a multiple of that): the aligned call's bits, nothing written beside them."""
+    import torch
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[ydt]
+    N = 64
+    pg, pu = (_packed(torch, Q4K, N, K, 941 + i, cuda)[1] for i in range(2))
+    x, _ = _act(torch, M, K, mx.BF16, 943, cuda)
+    try:
+        mx.qgemm.test_force_skinny(True)
+        y0 = mx.q_gemm_dequant(x, pg, M, N, K, Q4K, out_dtype=tdt, path=mx.PATH_MFMA)
+        h0 = mx.q_gemm_swiglu(x, pg, pu, out_dtype=tdt)
+        for off in (1, 2, 3):
+            for want in (y0, h0):
+                buf = torch.full((M * N + 8,), 7.5, dtype=tdt, device=cuda)
+                out = buf[off:off + M * N].view(M, N)
+                if want is y0:
+                    mx.q_gemm_dequant(x, pg, M, N, K, Q4K, out=out, path=mx.PATH_MFMA)
+                else:
+                    mx.q_gemm_swiglu(x, pg, pu, out=out)
+                torch.cuda.synchronize()
+                assert torch.equal(out, want), off
+                assert (buf[:off] == 7.5).all() and (buf[off + M * N:] == 7.5).all()
+    finally:
+        mx.qgemm.test_force_skinny(False)
+
+
 @pytest.mark.parametrize("qt,M", [(Q4K, 8), (Q80, 5), (Q6K, 3)])
 def test_skinny_staged_f16_activations_match_oracle(cuda, qt, M):
     """fp16 activations (the fp16 MFMA, fp16-rounded weights) through the staged narrow
