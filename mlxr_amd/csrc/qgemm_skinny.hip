@@ -29,10 +29,13 @@ const SkinnyKern& kern_for(int qtype, bool f16, int xr, int rt, int kg, bool sw,
 
 int rows_of_block(int M) { return M <= 8 ? 8 : M <= 16 ? 16 : 32; }
 
-// Workgroups of k a CU holds, asked once per device (with the LDS limit raised); 0: an error, in *e.
-int residents(const SkinnyKern& k, hipError_t* e) {
+int current_device() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  return hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 ? 0 : dev;
+}
+// Workgroups of k a CU of the current device holds, asked once per device (with the LDS limit
+// raised); 0: an error, in *e.
+int residents(const SkinnyKern& k, int dev, hipError_t* e) {
   int occ = k.residents[dev].load(std::memory_order_acquire);
   if (occ == 0) {
     if (k.lds > 65536) {
@@ -81,9 +84,9 @@ constexpr double kBytes[2][3] = {{3.57, 3.76, 3.98}, {3.71, 3.30, 4.09}};
 // us of a launch of `items` items of `turns` turns (kg = 1: super-blocks), `occ` workgroups on a CU.
 // Whole rounds of the device's workgroups, then the rest: the first workgroups, neighbours on an
 // XCD, take one item more.  The weights' bytes are read again, half from memory, by further blocks of M.
-double plan_us(int qtype, int xr, int rt, int kg, long items, long turns, int occ, int mblocks, double bytes) {
+double plan_us(int qtype, int xr, int rt, int kg, long items, long turns, int occ, long cus, int mblocks, double bytes) {
   const int x = xr == 8 ? 0 : xr == 16 ? 1 : 2, t = rt == 1 ? 0 : rt == 2 ? 1 : 2;
-  const long cus = device_cu_count(), slots = occ * cus;
+  const long slots = occ * cus;
   const long full = items / slots, rest = items % slots;
   const long n = full > 0 ? std::min<long>(occ, (rest + cus / 8 - 1) / (cus / 8)) : (rest + cus - 1) / cus;
   const TypeCost tc = type_cost(qtype);
@@ -116,7 +119,8 @@ Plan plan_for(const RunArgs* const* items, int n, bool swiglu) {
   const bool f16 = a.x_dtype == DT_F16;
   const int tiles = g_skinny_tiles.load(std::memory_order_relaxed), waves = g_skinny_waves.load(std::memory_order_relaxed),
             splits = g_skinny_splits.load(std::memory_order_relaxed);
-  const int nsb = (K + 255) / 256, turns = (nsb + 7) / 8;
+  const int nsb = (K + 255) / 256, turns = (nsb + 7) / 8, dev = current_device();
+  const long cus = device_cu_count();
   double bytes = 0;
   for (int i = 0; i < n; ++i) bytes += (double)items[i]->L.total;
   Plan best{0, 0, 0, 1e30};
@@ -125,10 +129,10 @@ Plan plan_for(const RunArgs* const* items, int n, bool swiglu) {
     long slabs = 0;
     for (int i = 0; i < (swiglu ? 1 : n); ++i) slabs += (items[i]->L.N + rows - 1) / rows;
     hipError_t e;
-    const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, kg, swiglu, ks > 1), &e));
+    const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, kg, swiglu, ks > 1), dev, &e));
     const long parts = (long)((M + xr - 1) / xr) * ks, nitems = slabs * parts;
     if (ks > 1 && (uint64_t)(nitems * parts) >= (1ull << 32)) return;
-    double us = plan_us(a.L.qtype, xr, rt, kg, nitems, kg == 1 ? nsb : (turns + ks - 1) / ks, occ,
+    double us = plan_us(a.L.qtype, xr, rt, kg, nitems, kg == 1 ? nsb : (turns + ks - 1) / ks, occ, cus,
                         (M + xr - 1) / xr, bytes);
     if (ks > 1) us += 3.1 + (double)ks * M * a.L.N * (swiglu ? 16 : 8) / 6.3e6;  // the second launch
     if (us < best.us) best = Plan{rt, kg, ks, us};
@@ -184,7 +188,7 @@ hipError_t launch_any(const RunArgs* const* items, int n, bool swiglu, hipStream
   sp.ws_split = (size_t)a.M * (size_t)sp.ws_ld;
   const SkinnyKern& k = kern_for(a.L.qtype, a.x_dtype == DT_F16, xr, pl.rt, pl.kg, swiglu, pl.ks > 1);
   hipError_t e = hipSuccess;
-  const int occ = residents(k, &e);
+  const int occ = residents(k, current_device(), &e);
   if (occ == 0) return e;
   const int nitems = slabs * sp.parts, grid = std::min(nitems, occ * device_cu_count());
   sp.per = nitems / grid;
