@@ -20,6 +20,15 @@ Q4K, Q6K, Q80 = mx.QuantType.Q4_K, mx.QuantType.Q6_K, mx.QuantType.Q8_0
 Q40, Q41, Q5K = mx.QuantType.Q4_0, mx.QuantType.Q4_1, mx.QuantType.Q5_K
 
 
+@pytest.fixture(params=["auto", "tiled"])
+def mfma_kernel(request):
+    """Calls of the MFMA family on the kernel of their choice, and on the tiled kernel (which the choice
+    gives few of the small shapes here)."""
+    mx.qgemm.test_force_tiled(request.param == "tiled")
+    yield request.param
+    mx.qgemm.test_force_tiled(False)
+
+
 def _dev_bytes(torch, arr, device):
     return torch.from_numpy(np.ascontiguousarray(arr)).to(device)
 
@@ -105,10 +114,10 @@ MFMA_CASES = [
     (Q41, 5, 64, 160),
     # tile edges with N % 4 != 0 (the epilogue's scalar stores) and ragged M
     (Q4K, 130, 250, 512), (Q6K, 300, 77, 256), (Q80, 200, 130, 1024),
-    # one wavefront per workgroup (short K) with two M-blocks: every row must be stored
+    # short K with M in two blocks: every row must be stored
     (Q4K, 40, 64, 256), (Q6K, 64, 32, 512), (Q80, 33, 64, 64),
     (Q5K, 128, 256, 1024), (Q5K, 9, 96, 768), (Q5K, 300, 200, 2048),
-    # the skinny kernel's narrow variant with one and two 16-row activation blocks
+    # one and two 16-row activation blocks of the skinny kernel
     (Q6K, 12, 200, 512), (Q6K, 24, 96, 768), (Q80, 30, 64, 1056), (Q40, 17, 130, 96), (Q5K, 32, 64, 256),
 ]
 
@@ -127,7 +136,7 @@ def test_gemv_lm_head_q6k_full_size(cuda):
 
 
 @pytest.mark.parametrize("qt,M,N,K", MFMA_CASES)
-def test_mfma_matches_oracle(cuda, qt, M, N, K):
+def test_mfma_matches_oracle(cuda, qt, M, N, K, mfma_kernel):
     import torch
     w, pw = _packed(torch, qt, N, K, 51 + M, cuda)
     x, xf = _act(torch, M, K, mx.BF16, 61 + N, cuda)
@@ -140,7 +149,7 @@ def test_mfma_matches_oracle(cuda, qt, M, N, K):
     assert orc.normwise_rel_err(y.cpu().numpy(), ref_exact) <= TOL  # normwise only: see rel_err
 
 
-def test_mfma_f16_activations(cuda):
+def test_mfma_f16_activations(cuda, mfma_kernel):
     import torch
     qt, M, N, K = Q4K, 160, 192, 1024
     w, pw = _packed(torch, qt, N, K, 71, cuda)
@@ -152,7 +161,7 @@ def test_mfma_f16_activations(cuda):
 
 @pytest.mark.parametrize("path", [mx.PATH_GEMV, mx.PATH_MFMA])
 @pytest.mark.parametrize("ydt", ["bf16", "f16", "f32"])
-def test_bias_and_output_dtypes(cuda, path, ydt):
+def test_bias_and_output_dtypes(cuda, path, ydt, mfma_kernel):
     import torch
     qt, M, N, K = Q4K, 4 if path == mx.PATH_GEMV else 136, 200, 512
     w, pw = _packed(torch, qt, N, K, 81, cuda)
@@ -196,8 +205,8 @@ def test_gemv_rows_independent_of_batch(cuda):
 
 @pytest.mark.parametrize("qt,M,N,K", [(Q4K, 512, 2048, 1024), (Q4K, 300, 1000, 512), (Q6K, 512, 1536, 768),
                                       (Q80, 512, 1536, 256)])
-def test_mfma_large_tile_matches_oracle(cuda, qt, M, N, K):
-    """Shapes with enough 256x256 tiles to take the large-tile kernel (ragged M and N too)."""
+def test_mfma_large_tile_matches_oracle(cuda, qt, M, N, K, mfma_kernel):
+    """Hundreds of rows on both sides, ragged M and N too."""
     import torch
     w, pw = _packed(torch, qt, N, K, 111 + M, cuda)
     x, xf = _act(torch, M, K, mx.BF16, 112 + N, cuda)
@@ -273,13 +282,22 @@ def test_swiglu_of_narrow_weights_takes_skinny_kernel(cuda, qt, M, N, K):
     assert ((h.double() - ref).abs() <= bound).all()
 
 
+def _assert_split(weights, M):
+    """A grouped call with the workspace asked for splits K on the tiled kernel."""
+    arr = (mx.qgemm.Item * len(weights))(*[mx.qgemm.Item(int(qt), N, K) for qt, N, K in weights])
+    need = ctypes.c_size_t(0)
+    assert mx.lib().mlxr_qgemm_grouped_workspace_size(len(weights), arr, M, ctypes.byref(need)) == 0
+    kernels = mx.qgemm.test_kernels("grouped_ws", weights, M, need.value)[0]
+    assert kernels == [mx.qgemm.KERNEL_TILED_SPLIT] * len(weights), kernels
+
+
 @pytest.mark.parametrize("M,K", [(65, 1024), (130, 4096), (300, 2048), (48, 4096)])
-def test_grouped_tiled_launches(cuda, M, K):
-    """Grouped calls on the tiled MFMA GEMM: same-type weights share one launch (tile columns
-    side by side).  Without a workspace the launch is unsplit and equals separate calls bit
-    for bit (M > 64); with the workspace the library asks for, the concatenated N may split
-    K (also for 32 < M <= 64) and stays within tolerance of the oracle, deterministically,
-    with a bias, a ragged N and a mixed-type group."""
+def test_grouped_tiled_launches(cuda, M, K, mfma_kernel):
+    """Grouped calls on the MFMA kernels: same-type weights share one launch (slabs or tile columns side
+    by side).  Without a workspace the launch is unsplit and equals separate calls bit for bit (M >
+    64); with the workspace the library asks for, a tiled launch splits the K of its concatenated
+    N (also for 32 < M <= 64) and stays within tolerance of the oracle, deterministically, with
+    a bias, a ragged N (the reduce's single columns) and a mixed-type group."""
     import torch
     specs = [(Q4K, 512), (Q4K, 130), (Q6K, 128), (Q4K, 640), (Q4K, 256)]
     gg = [mx.synth_gguf(qt, N, K, 300 + i) for i, (qt, N) in enumerate(specs)]
@@ -298,6 +316,8 @@ def test_grouped_tiled_launches(cuda, M, K):
                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
             assert rc == 0, L.mlxr_qgemm_last_error()
             assert torch.equal(y, y1), i
+    if mfma_kernel == "tiled" and K >= 2048:
+        _assert_split([(w.qtype, w.N, K) for w in ws], M)
     yw = mx.q_gemm_dequant_grouped(x, ws, biases=biases, out_dtype=torch.float32)
     yw2 = mx.q_gemm_dequant_grouped(x, ws, biases=biases, out_dtype=torch.float32)
     for i, (w, y, y2) in enumerate(zip(ws, yw, yw2)):
@@ -360,7 +380,7 @@ def test_grouped_without_workspace_equals_single_calls(cuda, specs, M, K):
 
 
 @pytest.mark.parametrize("ydt", ["bf16", "f32"])
-def test_grouped_split_reduce_vectorized(cuda, ydt):
+def test_grouped_split_reduce_vectorized(cuda, ydt, mfma_kernel):
     """Grouped tiled launch split over K whose weights all have N % 4 == 0 (the reduce then
     handles four columns per thread): within tolerance of the oracle with a bias on a middle
     weight, deterministic, for bf16 and f32 outputs."""
@@ -373,6 +393,8 @@ def test_grouped_split_reduce_vectorized(cuda, ydt):
     x, xf = _act(torch, M, K, mx.BF16, 510, cuda)
     bias = torch.linspace(-1, 1, 132, device=cuda).to(torch.bfloat16)
     biases = [None, bias, None]
+    if mfma_kernel == "tiled":
+        _assert_split([(Q4K, N, K) for N in Ns], M)
     ys = mx.q_gemm_dequant_grouped(x, ws, biases=biases, out_dtype=tdt)
     ys2 = mx.q_gemm_dequant_grouped(x, ws, biases=biases, out_dtype=tdt)
     for i, (y, y2) in enumerate(zip(ys, ys2)):
@@ -382,7 +404,7 @@ def test_grouped_split_reduce_vectorized(cuda, ydt):
         assert orc.rel_err(y.float().cpu().numpy(), ref) <= TOL, i
 
 
-def test_grouped_tiled_many_items_f16(cuda):
+def test_grouped_tiled_many_items_f16(cuda, mfma_kernel):
     """Five same-type weights (more than one launch holds: four, then one), fp16 activations
     and outputs, a K that ends on a half step (Q8_0, K % 64 == 32), with and without the
     workspace."""
@@ -405,9 +427,8 @@ def test_grouped_tiled_many_items_f16(cuda):
 
 @pytest.mark.parametrize("qt,M,N,K", [(Q4K, 300, 512, 4096), (Q6K, 256, 256, 2048), (Q80, 130, 384, 1056),
                                       (Q4K, 64, 1024, 14336)])
-def test_mfma_few_tiles_long_k(cuda, qt, M, N, K):
-    """Few output tiles (the 128-row tile variant) and long K, with bias; two calls in a
-    row agree bit for bit."""
+def test_mfma_few_tiles_long_k(cuda, qt, M, N, K, mfma_kernel):
+    """Few output tiles and long K, with bias; two calls in a row agree bit for bit."""
     import torch
     w, pw = _packed(torch, qt, N, K, 131 + M, cuda)
     x, xf = _act(torch, M, K, mx.BF16, 132 + N, cuda)
@@ -466,8 +487,8 @@ def test_skinny_operand_limit_falls_back_to_chunked_tiles(cuda, M):
     assert orc.rel_err(h.cpu().numpy(), g / (1.0 + np.exp(-g)) * u) <= TOL
 
 
-# The skinny kernel's narrow (16x16x32) variant on Q4_K: ragged N, K shorter than or not a
-# multiple of its ring (steps of 128), both activation dtypes, M from 1 to 16.
+# The skinny kernel on Q4_K: ragged N, K shorter than or not a multiple of the eight wavefronts'
+# super-blocks, both activation dtypes, M from 1 to 16.
 @pytest.mark.parametrize("M,N,K,xdt", [(5, 100, 768, mx.BF16), (8, 1000, 2304, mx.F16), (9, 257, 4096, mx.BF16),
                                        (16, 64, 256, mx.F16), (12, 30, 1280, mx.BF16), (1, 33, 512, mx.BF16),
                                        (16, 512, 14336, mx.BF16), (7, 4096, 1024, mx.F16)])
@@ -491,13 +512,13 @@ def test_skinny_q4k_matches_oracle(cuda, M, N, K, xdt):
                                           (Q4K, 8, 1024, 8192, "bf16"), (Q6K, 12, 2048, 4096, "f32"),
                                           (Q80, 5, 512, 2048, "f16"), (Q41, 16, 992, 4096, "bf16"),
                                           (Q80, 130, 384, 1056, "f16"), (Q4K, 2048, 1024, 4096, "f32")])
-def test_mfma_split_k(cuda, qt, M, N, K, ydt):
+def test_mfma_split_k(cuda, qt, M, N, K, ydt, mfma_kernel):
     """Split-K through the C ABI: mlxr_qgemm_run_ws with the workspace size the library
-    asks for splits K over workgroups (partials + reduce kernel: the skinny kernel for
-    M <= 32 with few 32-row slabs, the tiled kernel otherwise, with 64-row tiles
-    for 32 < M <= 64) and stays within tolerance of the oracle,
-    with bias, for every output dtype and N % 4 != 0; repeated calls are bit-identical, and
-    a workspace one byte too small gives exactly the unsplit mlxr_qgemm_run_ex result."""
+    asks for may split K over workgroups (partials + reduce kernel) and stays within tolerance of
+    the oracle, with bias, for every output dtype and N % 4 != 0; repeated calls are
+    bit-identical, and a workspace one byte too small gives exactly the unsplit
+    mlxr_qgemm_run_ex result.  Every shape here splits on the tiled kernel (16 splits at most;
+    64-row tiles at M <= 64), which writes the workspace then and not otherwise."""
     import ctypes
     import torch
     tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[ydt]
@@ -506,7 +527,11 @@ def test_mfma_split_k(cuda, qt, M, N, K, ydt):
     bias = torch.linspace(-1, 1, N, device=cuda).to(torch.bfloat16)
     wsb = mx.workspace_size(qt, N, K, M)
     assert wsb > 0 and wsb % (4 * M * N) == 0
-    ws = torch.empty(wsb, dtype=torch.uint8, device=cuda)
+    short = wsb - 1
+    if mfma_kernel == "tiled":
+        assert mx.qgemm.test_kernels("single", [(qt, N, K)], M, 16 * 4 * M * N)[0] == [mx.qgemm.KERNEL_TILED_SPLIT]
+        wsb, short = 16 * 4 * M * N, 4 * M * N
+    ws = torch.full((wsb,), 0x5A, dtype=torch.uint8, device=cuda)
     L = mx.lib()
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
@@ -519,7 +544,12 @@ def test_mfma_split_k(cuda, qt, M, N, K, ydt):
     ys = [torch.empty((M, N), dtype=tdt, device=cuda) for _ in range(4)]
     run(ys[0], ws.data_ptr(), wsb)
     run(ys[1], ws.data_ptr(), wsb)
-    run(ys[2], ws.data_ptr(), wsb - 1)
+    if mfma_kernel == "tiled":
+        assert (ws != 0x5A).any()
+        ws.fill_(0x5A)
+    run(ys[2], ws.data_ptr(), short)
+    if mfma_kernel == "tiled":
+        assert (ws == 0x5A).all()
     rc = L.mlxr_qgemm_run_ex(int(qt), N, K, 0, pw.data_ptr(), x.data_ptr(), mx.BF16, bias.data_ptr(), mx.BF16,
                              ys[3].data_ptr(), {"bf16": mx.BF16, "f16": mx.F16, "f32": mx.F32}[ydt], M,
                              mx.PATH_MFMA, s)
@@ -552,9 +582,8 @@ def test_python_binding_checks_outputs_and_bias(cuda):
     assert torch.equal(y, mx.q_gemm_dequant(x, pw, M, N, K, qt, out_dtype=torch.float32))
 
 
-# The 32x32x16 skinny kernel in 64-row blocks of M (second grid dimension), forced at
-# shapes the automatic choice may give the tiled kernel: ragged last M block, ragged N,
-# every type, K not a multiple of 64 (Q8_0, Q4_0), split K through the workspace.
+# The skinny kernel in several 32-row blocks of M, forced at shapes the choice may give the tiled
+# kernel: ragged last block, ragged N, every type, K not a multiple of 128 (Q8_0, Q4_0).
 @pytest.mark.parametrize("qt,M,N,K", [(Q4K, 65, 100, 768), (Q6K, 130, 257, 1024), (Q80, 200, 64, 1056),
                                       (Q40, 96, 33, 96), (Q41, 256, 128, 2048), (Q5K, 129, 96, 512),
                                       (Q4K, 300, 1024, 4096)])
@@ -573,17 +602,13 @@ def test_skinny_m_blocks_match_oracle(cuda, qt, M, N, K):
     assert torch.equal(y, y2)
     ref = orc.gemm_f64(int(qt), M, N, K, w, xf, bias=bias.float().cpu().numpy(), w_to_bf16=True)
     err = orc.rel_err(y.cpu().numpy(), ref)
-    # same bf16 weights as the oracle: only the fp32 accumulation order differs (K up to
-    # 4096 in up to eight split partials)
+    # same bf16 weights as the oracle: only the fp32 accumulation order differs
     assert err <= 3e-5, err
 
 
-# Shapes whose narrow-kernel plan stages the activations in LDS (M <= 8, eight or more steps
-# per wavefront): Llama-3-8B gate, ragged N with a bias and half-precision outputs, K not a
-# multiple of the 128-wide step (Q4_0, Q8_0), M <= 4 through the MFMA path, down shapes (K
-# split over two workgroups, seven wavefronts of 112 KiB of stages), long stages at M = 1
-# and 2 (32 and 16 steps per wavefront), M = 9 to 16 (two slabs per workgroup sharing their
-# stages; 14300 rows: an odd slab count, the last workgroup's second slab past N).
+# Shapes of whole layers at M <= 16: Llama-3-8B gate, ragged N with a bias and half-precision outputs, K
+# not a multiple of the 128-wide step (Q4_0, Q8_0), M <= 4 through the MFMA path, down shapes, long
+# rows at M = 1 and 2, thousands of rows that end inside a tile.
 @pytest.mark.parametrize("qt,M,N,K,path,ydt", [(Q4K, 8, 14336, 4096, mx.PATH_AUTO, "f32"),
                                                (Q6K, 6, 14000, 4096, mx.PATH_AUTO, "bf16"),
                                                (Q80, 5, 11008, 4000, mx.PATH_AUTO, "f16"),
@@ -600,11 +625,8 @@ def test_skinny_m_blocks_match_oracle(cuda, qt, M, N, K):
                                                (Q41, 13, 11001, 4096, mx.PATH_AUTO, "f32"),
                                                (Q4K, 12, 14300, 4096, mx.PATH_AUTO, "bf16")])
 def test_skinny_staged_activations_match_oracle(cuda, qt, M, N, K, path, ydt):
-    """The narrow skinny kernel with its activations staged in LDS (one slab per workgroup
-    where that fits, two slabs sharing their stages otherwise or when preferred through the
-    test hook) gives the same bits as the kernel reading them from global memory (same
-    products in the same order), and all agree with the oracle over the bf16-rounded
-    weights."""
+    """One, two and four weight tiles per wavefront, and the choice by shape, give the same bits (the same
+    products in the same order), and all agree with the oracle over the bf16-rounded weights."""
     import torch
     w, pw = _packed(torch, qt, N, K, 211 + M, cuda)
     x, xf = _act(torch, M, K, mx.BF16, 221 + M, cuda)
@@ -612,14 +634,14 @@ def test_skinny_staged_activations_match_oracle(cuda, qt, M, N, K, path, ydt):
     tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[ydt]
     ys = {}
     try:
-        for mode in (1, 2, 0):
+        for mode in (1, 2, 0, 4):
             mx.qgemm.test_skinny_stage(mode)
             ys[mode] = mx.q_gemm_dequant(x, pw, M, N, K, qt, bias=bias, out_dtype=tdt, path=path)
     finally:
         mx.qgemm.test_skinny_stage(1)
     torch.cuda.synchronize()
-    assert torch.equal(ys[1], ys[0])
-    assert torch.equal(ys[2], ys[0])
+    for mode in (1, 2, 4):
+        assert torch.equal(ys[mode], ys[0]), mode
     ref = orc.gemm_f64(int(qt), M, N, K, w, xf, bias=bias.float().cpu().numpy(), w_to_bf16=True)
     # half-precision outputs add their own rounding (2^-9 / 2^-12 relative)
     assert orc.rel_err(ys[1].float().cpu().numpy(), ref) <= (5e-3 if ydt != "f32" else 3e-5)
@@ -827,11 +849,64 @@ def test_skinny_outputs_at_any_element_address(cuda, ydt, M, K):
         mx.qgemm.test_force_skinny(False)
 
 
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("qt,M,N,K", [(Q4K, 33, 300, 4096), (Q6K, 100, 129, 2048), (Q80, 300, 130, 1056), (Q5K, 8, 64, 512)])
+def test_tiled_swiglu_matches_oracle(cuda, qt, M, N, K, workspace):
+    """The fused SwiGLU on the tiled kernel, unsplit and (with its workspace) split over K: ragged M and N,
+    K that ends inside a step."""
+    import torch
+    (wg, pg), (wu, pu) = _packed(torch, qt, N, K, 951, cuda), _packed(torch, qt, N, K, 952, cuda)
+    x, xf = _act(torch, M, K, mx.BF16, 953 + M, cuda)
+    try:
+        mx.qgemm.test_force_tiled(True)
+        v = ctypes.c_size_t(0)
+        assert mx.lib().mlxr_qgemm_swiglu_workspace_size(int(qt), N, K, M, mx.F32, ctypes.byref(v)) == 0
+        served = mx.qgemm.test_kernels("swiglu", [(qt, N, K)], M, v.value if workspace else 0)[0][0]
+        assert served == (mx.qgemm.KERNEL_TILED_SPLIT if workspace and M > 32 else mx.qgemm.KERNEL_TILED)
+        h = mx.q_gemm_swiglu(x, pg, pu, out_dtype=torch.float32, workspace=workspace)
+    finally:
+        mx.qgemm.test_force_tiled(False)
+    g, u = (orc.gemm_f64(int(qt), M, N, K, w, xf, w_to_bf16=True).astype(np.float64) for w in (wg, wu))
+    assert orc.rel_err(h.cpu().numpy(), g / (1.0 + np.exp(-g)) * u) <= TOL
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 4])
+@pytest.mark.parametrize("qt,M,N,K", [(Q4K, 70, 9003, 2304), (Q6K, 13, 20000, 512), (Q80, 100, 12290, 1056)])
+def test_skinny_workgroups_walk_several_items(cuda, qt, M, N, K, tiles):
+    """More items than workgroups fit the device, so each walks several (next weight rows, next block of M,
+    next weight of a grouped launch), with blocks of M that are no power of two: a grouped call and
+    the fused SwiGLU against the products of the library's dequantized weights in fp64, with the bound of
+    test_skinny_tile_counts_match_oracle."""
+    import torch
+    pws = [_packed(torch, qt, N, K, 961 + i, cuda)[1] for i in range(2)]
+    x, _ = _act(torch, M, K, mx.BF16, 963 + M, cuda)
+    try:
+        mx.qgemm.test_force_skinny(True)
+        mx.qgemm.test_skinny_plan(tiles, 8)
+        ys = mx.q_gemm_dequant_grouped(x, pws, out_dtype=torch.float32)
+        h = mx.q_gemm_swiglu(x, *pws, out_dtype=torch.float32)
+    finally:
+        mx.qgemm.test_skinny_plan()
+        mx.qgemm.test_force_skinny(False)
+    terms = (32 + 8 + K // 2048 + 1 + 8) * 2.0**-23
+    xd, refs, errs = x.double(), [], []
+    for pw, y in zip(pws, ys):
+        w = mx.dequantize(pw, torch.bfloat16).double()
+        refs.append(xd @ w.T)
+        errs.append(xd.abs() @ w.abs().T * terms)
+        assert ((y.double() - refs[-1]).abs() <= errs[-1] + 2.0**-24 * refs[-1].abs()).all()
+    g, u = refs
+    sw = g * torch.sigmoid(g)
+    bound = 1.1 * errs[0] * (u.abs() + errs[1]) + sw.abs() * errs[1] + (16 + 2 * g.abs()) * 2.0**-23 * (sw * u).abs() \
+        + 2.0**-126 * (1 + u.abs())
+    assert ((h.double() - sw * u).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("qt,M", [(Q4K, 8), (Q80, 5), (Q6K, 3)])
 def test_skinny_staged_f16_activations_match_oracle(cuda, qt, M):
-    """fp16 activations (the fp16 MFMA, fp16-rounded weights) through the staged narrow
-    kernel on the Llama-3-8B gate shape: same bits as the global-read mode, within 3e-5 of
-    the oracle over the fp16-rounded weights."""
+    """fp16 activations (the fp16 MFMA, fp16-rounded weights) on the Llama-3-8B gate shape: same bits
+    with the tiles chosen by shape and with one, within 3e-5 of the oracle over the fp16-rounded
+    weights."""
     import torch
     N, K = 14336, 4096
     w, pw = _packed(torch, qt, N, K, 281 + M, cuda)
@@ -851,9 +926,8 @@ def test_skinny_staged_f16_activations_match_oracle(cuda, qt, M):
 
 @pytest.mark.parametrize("M", [6, 8, 16])
 def test_skinny_staged_swiglu_matches_oracle(cuda, M):
-    """Fused SwiGLU through the staged narrow kernel (16-row slabs of gate and up, 512 of
-    them: N = 8192 at K = 4096): same bits as the global-read mode, and the oracle's
-    swish(g) * u within 5e-3."""
+    """Fused SwiGLU on the skinny kernel (N = 8192 at K = 4096): same bits with two and four tiles per
+    wavefront and by shape, and the oracle's swish(g) * u within 5e-3."""
     import torch
     qt, N, K = Q4K, 8192, 4096
     wg, pg = _packed(torch, qt, N, K, 231, cuda)
@@ -861,14 +935,14 @@ def test_skinny_staged_swiglu_matches_oracle(cuda, M):
     x, xf = _act(torch, M, K, mx.BF16, 233 + M, cuda)
     hs = {}
     try:
-        for mode in (1, 2, 0):
+        for mode in (1, 2, 4):
             mx.qgemm.test_skinny_stage(mode)
             hs[mode] = mx.q_gemm_swiglu(x, pg, pu, out_dtype=torch.float32)
     finally:
         mx.qgemm.test_skinny_stage(1)
     torch.cuda.synchronize()
-    assert torch.equal(hs[1], hs[0])
-    assert torch.equal(hs[2], hs[0])
+    assert torch.equal(hs[1], hs[2])
+    assert torch.equal(hs[4], hs[2])
     g = orc.gemm_f64(int(qt), M, N, K, wg, xf, w_to_bf16=True).astype(np.float64)
     u = orc.gemm_f64(int(qt), M, N, K, wu, xf, w_to_bf16=True).astype(np.float64)
     assert orc.rel_err(hs[1].cpu().numpy(), g / (1.0 + np.exp(-g)) * u) <= 5e-3
@@ -937,9 +1011,8 @@ def test_grouped_call_at_small_m_with_large_weights(cuda, M):
 
 @pytest.mark.parametrize("qt,N,K", [(Q4K, 1024, 4096), (Q6K, 4096, 4096)])
 def test_narrow_weights_at_mid_m_take_skinny_kernel(cuda, qt, N, K):
-    """Shapes at M = 128 whose estimated times favour the skinny kernel: Llama-3-8B k (the
-    skinny kernel splits K, so it asks for a workspace) and a Q6_K 4096x4096 weight (256
-    blocks fill the device: workspace size 0).  With the workspace the library asks for the
+    """Shapes at M = 128 whose estimated times favour the skinny kernel: Llama-3-8B k (a workspace is
+    asked for) and a Q6_K 4096x4096 weight (workspace size 0).  With the workspace the library asks for the
     call is bit-equal to the forced skinny call; mlxr_qgemm_run_ex without a workspace makes
     the same choice when the size is 0 and otherwise runs the tiled kernel unsplit; all
     within tolerance of the oracle."""
@@ -969,7 +1042,7 @@ def test_narrow_weights_at_mid_m_take_skinny_kernel(cuda, qt, N, K):
 
 def test_concurrent_calls_from_host_threads(cuda):
     """Four host threads, each with its own stream and workspace, issue calls of every kernel
-    family (GEMV, staged and unstaged skinny, tiled split-K) at once; every output equals the
+    family (GEMV, skinny, tiled) at once; every output equals the
     same call made alone, bit for bit (the library's per-device caches and per-thread error
     strings are shared state)."""
     import threading

@@ -144,10 +144,9 @@ def test_random_swiglu_matches_oracle(cuda, seed):
 
 @pytest.mark.parametrize("seed", list(range(16)))
 def test_random_staged_skinny_call_matches_oracle(cuda, seed):
-    """Random shapes in the range where the narrow skinny kernel stages its activations in
-    LDS (M <= 8 through the MFMA path, thousands of rows, K of 4096 or a little less or more):
-    the staged call gives the same bits as the global-read one, and both are within the
-    contract of the oracle over the bf16-rounded weights."""
+    """Random shapes of decode (M <= 8 through the MFMA path, thousands of rows, K of 4096 or a little less
+    or more): the skinny kernel gives the same bits with the tiles chosen by shape and with one
+    per wavefront, within the contract of the oracle over the bf16-rounded weights."""
     import torch
     rng = np.random.default_rng(12000 + seed)
     qt = TYPES[int(rng.integers(len(TYPES)))]

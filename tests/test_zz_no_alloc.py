@@ -47,9 +47,14 @@ def test_noalloc_equals_workspace_entry_point(cuda):
     pw = mx.pack_weights(w, N, K, Q4K, device=cuda)
     ws = torch.empty(SCRATCH, dtype=torch.uint8, device=cuda)
     # first call: prefill rows whose tiled launch splits K; second: a smaller batched-decode
-    # input whose skinny launch splits K too (down shape), so the array is reused
-    cases = [(N, K, 512, pw, 11), (4096, 14336, 8, None, 12)]
-    for N_, K_, M, p, seed in cases:
+    # input whose skinny launch splits K too (few rows, long K), so the array is reused; third: a
+    # tiled split again
+    cases = [(N, K, 512, pw, 11), (1024, 14336, 8, None, 12), (4096, 14336, 100, None, 14)]
+    tiled, skinny = qgemm.KERNEL_TILED_SPLIT, qgemm.KERNEL_SKINNY
+    for (N_, K_, M, p, seed), kernel in zip(cases, (tiled, skinny, tiled)):
+        assert qgemm.test_kernels("single", [(Q4K, N_, K_)], M, SCRATCH)[0] == [kernel]
+        if kernel == skinny:
+            assert qgemm.test_skinny_layout(Q4K, N_, K_, M, False, _need(N_, K_, M))[2] > 1
         if p is None:
             p = mx.pack_weights(mx.synth_gguf(Q4K, N_, K_, 6), N_, K_, Q4K, device=cuda)
         need = _need(N_, K_, M)
