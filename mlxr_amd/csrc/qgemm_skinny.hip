@@ -171,6 +171,8 @@ hipError_t launch_any(const RunArgs* const* items, int n, bool swiglu, hipStream
     g.slab0 = slabs;
     g.y_dtype = b.y_dtype;
     g.bias_dtype = b.bias_dtype;
+    const bool f32 = pl.ks > 1 || b.y_dtype == DT_F32;
+    g.wide = (b.L.N & 3) == 0 && ((uintptr_t)(pl.ks > 1 ? a.ws : b.y) & (f32 ? 15u : 7u)) == 0;
     if (i < (swiglu ? 1 : n)) slabs += (b.L.N + rows - 1) / rows;
     if (swiglu) g.slab0 = 0;
   }

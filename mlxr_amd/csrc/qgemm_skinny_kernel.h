@@ -51,6 +51,7 @@ struct SkinnyGroup {
   int N;
   int slab0;  // first slab of this weight in the launch
   int y_dtype, bias_dtype;
+  int wide;  // y's address (split: ws's) and rows are aligned to four outputs
 };
 struct SkinnyParams {
   const void* x;
@@ -105,12 +106,12 @@ __device__ __forceinline__ void decode_hdr1(const Hdr<QT>& h, uint32_t sel, Scal
   }
 }
 
-// Four consecutive outputs of one row, in one store where y's address and rows are aligned to it.
-__device__ __forceinline__ void store4(void* y, int y_dtype, size_t rowbase, int nn, int N, const f32x4_t& v) {
+// Four consecutive outputs of one row, in one store where they are aligned to it.
+__device__ __forceinline__ void store4(void* y, int y_dtype, bool wide, size_t rowbase, int nn, int N, const f32x4_t& v) {
   const uint2 h = y_dtype == DT_BF16 ? make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]))
                                      : make_uint2(pack2<X_F16>(v[0], v[1]), pack2<X_F16>(v[2], v[3]));
   const size_t at = rowbase + nn;
-  if ((N & 3) == 0 && ((uintptr_t)y & (y_dtype == DT_F32 ? 15 : 7)) == 0 && nn + 3 < N) {
+  if (wide && nn + 3 < N) {
     if (y_dtype == DT_F32) *(f32x4_t*)((float*)y + at) = v;
     else *(uint2*)((uint16_t*)y + at) = h;
   } else {
@@ -389,8 +390,8 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG, SPLIT>())) voi
       if constexpr (SPLIT) {  // this split's partial sums, no bias
         float* const w = p.ws + (size_t)split_of(sub) * p.ws_split + (size_t)m * p.ws_ld;
         if (m < M) {
-          store4(w, DT_F32, 0, nn, N, sum);
-          if constexpr (SW) store4(w + N, DT_F32, 0, nn, N, up);
+          store4(w, DT_F32, G.wide, 0, nn, N, sum);
+          if constexpr (SW) store4(w + N, DT_F32, G.wide, 0, nn, N, up);
         }
         return;
       }
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(64 * KG, (skinny_occ<QT, XR, RT, KG, SPLIT>())) voi
         for (int e = 0; e < 4; ++e)
           if (nn + e < N) sum[e] += load_scalar(G.bias, G.bias_dtype, nn + e);
       }
-      if (m < M) store4(G.y, G.y_dtype, (size_t)m * N, nn, N, sum);
+      if (m < M) store4(G.y, G.y_dtype, G.wide, (size_t)m * N, nn, N, sum);
     };
     if constexpr (KG == 1) {
       sfor<HT * NB>([&](auto U_) {
@@ -547,7 +548,7 @@ const SkinnyKern& kern_of(int xr, int rt, int kg, bool sw, bool split) {
 
 // One translation unit per quant type instantiates the kernels (qgemm_skinny_<type>.hip).  xr: rows
 // of a block of M (8, 16, 32); rt: tiles per wavefront (1, 2, 4; SwiGLU 2, 4); kg: wavefronts (8, or
-// 1 for K <= 2048); split: K split over workgroups (kg = 8 and the fewest tiles).
+// 1 for K <= 1024); split: K split over workgroups (kg = 8 and the fewest tiles).
 const SkinnyKern& kern_q4k(bool f16, int xr, int rt, int kg, bool sw, bool split);
 const SkinnyKern& kern_q6k(bool f16, int xr, int rt, int kg, bool sw, bool split);
 const SkinnyKern& kern_q5k(bool f16, int xr, int rt, int kg, bool sw, bool split);
