@@ -65,12 +65,10 @@ std::atomic<int> g_forced{kNotForced};
 int forced() { return g_forced.load(std::memory_order_relaxed); }
 
 // Whether the skinny kernel is estimated to be ahead of the tiled one, which takes the weights as one
-// of `cols` columns with a workspace of ws_bytes.  The estimates are 7% off on average: where
-// they are within 5% of each other the tiled kernel stays (Q4_K SwiGLU 8192 x 3072 at M = 64, us,
-// skinny / tiled: estimated 24.9 / 25.5, measured 27.2 / 24.2).
+// of `cols` columns with a workspace of ws_bytes.
 bool skinny_ahead(const mlxr::RunArgs* const* items, int n, bool swiglu, int cols, size_t ws_bytes) {
   const mlxr::RunArgs& a = *items[0];
-  return mlxr::skinny_us(items, n, swiglu) < 0.95 * mlxr::mfma_us(a.M, cols, a.L.K, a.L.qtype, ws_bytes);
+  return mlxr::skinny_us(items, n, swiglu) < mlxr::mfma_us(a.M, cols, a.L.K, a.L.qtype, swiglu, ws_bytes);
 }
 
 // The kernel of a single call: GEMV (no MFMA) for decode (gemv_auto); MFMA kernels otherwise, the

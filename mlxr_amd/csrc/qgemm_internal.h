@@ -97,9 +97,9 @@ size_t skinny_workspace_bytes(int M, int N, int K, int qtype);
 // because callers size their buffers by the result; they choose no kernel.
 double skinny_sizing_us(int M, int N, int K);
 double mfma_sizing_us(int M, int N, int K, int qtype);
-// Estimated time in microseconds of the tiled kernel over an [M, N, K] problem that has a workspace
-// of ws_bytes, of its launch and the reduce.
-double mfma_us(int M, int N, int K, int qtype, size_t ws_bytes);
+// Estimated time in microseconds of the tiled kernel over an [M, N, K] problem (swiglu: N of gate and
+// up) that has a workspace of ws_bytes, of its launch and the reduce.
+double mfma_us(int M, int N, int K, int qtype, bool swiglu, size_t ws_bytes);
 // SwiGLU, h = swish(x.gate^T + bias_g) * (x.up^T + bias_u) into gate.y, with gate and up
 // of one type and shape; gate.ws / ws (may be null) holds split-K partials.
 // Skinny kernel and tiled kernel (any M; operands below 2 GiB, mfma_groupable; no biases).

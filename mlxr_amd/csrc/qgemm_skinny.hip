@@ -56,48 +56,56 @@ struct Plan {
   double us;
 };
 
-// Measured on MI355X by 15000 launches over [512 .. 128256] x [256 .. 28672] at M = 5 .. 128, all
-// types, weights from memory (7% off on average; the variant chosen by it 0.2% slower than the best
-// one on average, 1% or less for 95%).  us of a turn (one super-block for each of eight
-// wavefronts) of a workgroup, by rows of X (8, 16, 32) and tiles (1, 2, 4), Q4_K; the workgroups of
-// a CU take as many.  A lone wavefront's super-block takes kLoneLat + n * kLoneCu on a CU of n.  The
-// other types by their dequantization.
-constexpr double kTurn[3][3] = {{1.25, 2.31, 4.20}, {1.64, 2.62, 4.52}, {2.32, 3.27, 5.22}};
-constexpr double kLoneLat[3][3] = {{0.63, 1.43, 2.46}, {0.73, 1.47, 2.63}, {0.87, 1.77, 3.14}};
-constexpr double kLoneCu[3][3] = {{0.10, 0.07, 0.26}, {0.12, 0.13, 0.24}, {0.18, 0.20, 0.35}};
+// Fitted to 17000 launches measured on MI355X (36 shapes of [512 .. 65536] x [512 .. 28672], fused SwiGLU of
+// 12, M = 6 .. 2048, all types, weights from memory), to the times and to what the choices by them
+// lose: 5% off on average; the variant chosen, tiled kernel included, is 0.15% slower than the best
+// on average and more than 5% slower for 1% of the shapes.  us of a turn (one super-block for each
+// of eight wavefronts) of a workgroup, by rows of X (8, 16, 32) and tiles (1, 2, 4), Q4_K; the
+// workgroups of a CU take as many.  A lone wavefront's super-block takes kLoneLat + n * kLoneCu on a
+// CU of n.  The other types by their dequantization.
+constexpr double kTurn[3][3] = {{1.063, 2.184, 3.945}, {1.370, 2.437, 4.345}, {1.987, 2.910, 5.014}};
+constexpr double kLoneLat[3][3] = {{0.421, 0.830, 2.321}, {0.534, 1.080, 2.314}, {0.698, 1.308, 2.071}};
+constexpr double kLoneCu[3][3] = {{0.064, 0.220, 0.132}, {0.034, 0.133, 0.172}, {0.108, 0.170, 0.488}};
 struct TypeCost {
   double turn[3], lone;
 };
 TypeCost type_cost(int qtype) {
   switch (qtype) {
-    case QT_Q5_K: return {{1.13, 1.23, 1.26}, 1.19};
-    case QT_Q6_K: return {{1.19, 1.30, 1.35}, 1.22};
-    case QT_Q8_0: return {{1.11, 1.15, 1.16}, 1.02};
-    case QT_Q4_0: return {{0.98, 0.99, 1.00}, 0.94};
-    case QT_Q4_1: return {{0.99, 1.00, 1.01}, 0.95};
+    case QT_Q5_K: return {{1.115, 1.202, 1.212}, 1.200};
+    case QT_Q6_K: return {{1.202, 1.295, 1.293}, 1.265};
+    case QT_Q8_0: return {{1.092, 1.108, 1.120}, 1.045};
+    case QT_Q4_0: return {{0.946, 0.937, 0.964}, 0.909};
+    case QT_Q4_1: return {{0.945, 0.946, 0.975}, 0.892};
     default: return {{1.0, 1.0, 1.0}, 1.0};
   }
 }
-// What the weights' bytes take, MB/us (TB/s), by tiles: eight wavefronts, a lone one.
-constexpr double kBytes[2][3] = {{3.57, 3.76, 3.98}, {3.71, 3.30, 4.09}};
+// What the weights' bytes take, MB/us (TB/s), by tiles (Q8_0, whose rows are read in 32-byte pieces,
+// 1.31 times that), and the activations, read by every item: eight wavefronts, a lone one.
+constexpr double kBytes[2][3] = {{4.113, 4.547, 4.693}, {4.521, 4.541, 11.461}};
+constexpr double kXBytes[2] = {32.2, 15.5};
 
 // us of a launch of `items` items of `turns` turns (kg = 1: super-blocks), `occ` workgroups on a CU.
 // Whole rounds of the device's workgroups, then the rest: the first workgroups, neighbours on an
-// XCD, take one item more.  The weights' bytes are read again, half from memory, by further blocks of M.
-double plan_us(int qtype, int xr, int rt, int kg, long items, long turns, int occ, long cus, int mblocks, double bytes) {
+// XCD, take one item more.  A part of the weights' bytes is read from memory again by each further
+// block of M.
+double plan_us(int qtype, int xr, int rt, int kg, long items, long turns, int occ, long cus, int mblocks, double bytes,
+               double xbytes) {
   const int x = xr == 8 ? 0 : xr == 16 ? 1 : 2, t = rt == 1 ? 0 : rt == 2 ? 1 : 2;
   const long slots = occ * cus;
   const long full = items / slots, rest = items % slots;
   const long n = full > 0 ? std::min<long>(occ, (rest + cus / 8 - 1) / (cus / 8)) : (rest + cus - 1) / cus;
   const TypeCost tc = type_cost(qtype);
-  auto dur = [&](long n) {
-    if (n == 0) return 0.0;
-    return kg == 1 ? turns * (kLoneLat[x][t] + kLoneCu[x][t] * n) * tc.lone
-                   : turns * kTurn[x][t] * tc.turn[t] * (n + 0.1) / 1.1 + 0.3;
-  };
-  const double c = kg == 1 ? 2.8 : 2.6;
-  const double a = c + full * dur(occ) + dur(n);
-  const double m = c + bytes * (0.5 + 0.5 * mblocks) * 1e-6 / kBytes[kg == 1][t];
+  double a, m;
+  if (kg == 1) {
+    auto dur = [&](long n) { return n ? turns * (kLoneLat[x][t] + kLoneCu[x][t] * n) * tc.lone + 3.7 : 0.0; };
+    // items after the first of their workgroup start with their operands loaded
+    a = full > 0 ? dur(occ) + 0.73 * ((full - 1) * dur(occ) + dur(n)) : dur(n);
+    m = (bytes * (0.81 + 0.19 * mblocks) / kBytes[1][t] + xbytes / kXBytes[1]) * 1e-6;
+  } else {
+    auto dur = [&](long n) { return n ? turns * kTurn[x][t] * tc.turn[t] * n + 0.74 : 0.0; };
+    a = 2.67 + full * dur(occ) + dur(n);
+    m = 2.67 + (bytes * (0.68 + 0.32 * mblocks) / (kBytes[0][t] * (qtype == QT_Q8_0 ? 1.31 : 1.0)) + xbytes / kXBytes[0]) * 1e-6;
+  }
   return std::sqrt(std::sqrt(a * a * a * a + m * m * m * m));
 }
 
@@ -132,8 +140,9 @@ Plan plan_for(const RunArgs* const* items, int n, bool swiglu) {
     const int occ = std::max(1, residents(kern_for(a.L.qtype, f16, xr, rt, kg, swiglu, ks > 1), dev, &e));
     const long parts = (long)((M + xr - 1) / xr) * ks, nitems = slabs * parts;
     if (ks > 1 && (uint64_t)(nitems * parts) >= (1ull << 32)) return;
-    double us = plan_us(a.L.qtype, xr, rt, kg, nitems, kg == 1 ? nsb : (turns + ks - 1) / ks, occ, cus,
-                        (M + xr - 1) / xr, bytes);
+    const int mblocks = (M + xr - 1) / xr;
+    double us = plan_us(a.L.qtype, xr, rt, kg, nitems, kg == 1 ? nsb : (turns + ks - 1) / ks, occ, cus, mblocks, bytes,
+                        2.0 * slabs * mblocks * xr * K);
     if (ks > 1) us += 3.1 + (double)ks * M * a.L.N * (swiglu ? 16 : 8) / 6.3e6;  // the second launch
     if (us < best.us) best = Plan{rt, kg, ks, us};
   };

@@ -474,28 +474,27 @@ double mfma_sizing_us(int M, int N, int K, int qtype) {
   return t * 1.86 + (sp.kps <= 8 && nkt > 8 ? 4.5 : 0.0);
 }
 
-// Measured on MI355X over 21 shapes of ordinary models at M = 33 .. 2048, all types, split and
-// not, SwiGLU as 2N columns (7% off on average): us of a step of 256-, 128- and 64-row tiles, Q4_K,
-// and what the other types' dequantization makes of it (past the first steps, which wait for memory); 8 us per round of workgroups beside its
-// steps, of which a round that fills a part of the CUs saves a sixth of the empty part; the reduce
-// launch.
-double mfma_us(int M, int N, int K, int qtype, size_t ws_bytes) {
+// Fitted with the skinny kernel's estimate (2600 of the launches, M = 33 .. 2048, split and not): us of a
+// step of 256-, 128- and 64-row tiles, Q4_K, and what the other types' dequantization and the fused
+// SwiGLU (of 2N columns) make of it; what a round of workgroups takes beside its steps, of which one
+// that fills a part of the CUs saves 0.14 of the empty part; the reduce launch.
+double mfma_us(int M, int N, int K, int qtype, bool swiglu, size_t ws_bytes) {
   SplitPlan sp = plan_split(M, N, K, ~(size_t)0);
   if (sp.S > 1 && (size_t)sp.S * (size_t)M * (size_t)N * 4u > ws_bytes) sp = plan_split(M, N, K, 0);
-  constexpr double kStep[3] = {1.55, 0.89, 0.66};
-  static const double kType[4][3] = {{1, 1, 1}, {1.13, 1.28, 1.46}, {1.17, 1.32, 1.52}, {1.11, 1.30, 1.55}};
+  constexpr double kStep[3] = {1.545, 0.816, 0.640}, kSwiglu[3] = {0.938, 0.944, 0.871}, kRound[3] = {9.57, 10.5, 7.89};
+  constexpr double kType[6][3] = {{1, 1, 1},             {1.149, 1.393, 1.463}, {1.200, 1.399, 1.579},
+                                  {1.139, 1.336, 1.485}, {1.007, 1.042, 1.109}, {1.016, 1.057, 1.120}};
   const int b = sp.bm == 256 ? 0 : sp.bm == 128 ? 1 : 2;
-  const int t = qtype == QT_Q5_K ? 1 : qtype == QT_Q6_K ? 2 : qtype == QT_Q8_0 ? 3 : 0;
-  const double q4 = qtype == QT_Q4_0 || qtype == QT_Q4_1 ? 1.0 + 0.06 * b : 1.0;
+  const int t = qtype == QT_Q5_K ? 1 : qtype == QT_Q6_K ? 2 : qtype == QT_Q8_0 ? 3 : qtype == QT_Q4_0 ? 4 : qtype == QT_Q4_1 ? 5 : 0;
   const int cus = device_cu_count(), ring = qtype == QT_Q8_0 ? 4 : 8;
   const int steps = ((sp.S > 1 ? sp.kps : (K + TK - 1) / TK) + ring - 1) / ring * ring;
   const long wgs = (long)sp.tiles * sp.S;
-  const double part = (double)(wgs % cus) / cus;
-  const double round = steps * kStep[b] + std::max(steps - 6, 0) * kStep[b] * (kType[t][b] * q4 - 1.0) + 8.0;
-  double us = (wgs / cus + (part > 0 ? 0.84 + 0.16 * part : 0)) * round;
-  if (sp.S > 1) us += 3.8 + (double)sp.S * M * N * 8.0 / 6.4e6;
-  // operands at 3 TB/s
-  const double m = ((double)N * K * gguf_block_bytes(qtype) / gguf_block_elems(qtype) + 2.0 * M * ((double)N + K)) / 3e6;
+  const double part = (double)(wgs % cus) / cus, step = kStep[b] * kType[t][b] * (swiglu ? kSwiglu[b] : 1.0);
+  double us = (wgs / cus + (part > 0 ? 0.86 + 0.14 * part : 0)) * (steps * step + kRound[b]);
+  if (sp.S > 1) us += 5.5 + (double)sp.S * M * N * 8.0 / 12e6;
+  // operands at 2.8 TB/s
+  const double w = (double)N * K * gguf_block_bytes(qtype) / gguf_block_elems(qtype) / (qtype == QT_Q8_0 ? 1.28 : 1.0);
+  const double m = (w + 2.0 * M * ((double)N + K)) / 2.81e6;
   return std::sqrt(std::sqrt(us * us * us * us + m * m * m * m));
 }
 

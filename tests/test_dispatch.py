@@ -89,6 +89,13 @@ MEASURED = [
     ("single", [(Q4K, 4096, 4096)], 64, "skinny", 10.7, 18.1),
     ("single", [(Q4K, 5120, 5120)], 33, "skinny", 18.7, 59.8),
     ("single", [(Q4K, 3072, 8192)], 64, "skinny", 16.9, 26.3),
+    ("single", [(Q80, 8192, 8192)], 48, "skinny", 29.2, 36.2),
+    ("single", [(Q80, 8192, 8192)], 64, "skinny", 31.1, 35.7),
+    ("single", [(Q5K, 5120, 5120)], 64, "skinny", 22.8, 25.3),
+    ("single", [(Q4K, 3072, 8192)], 96, "skinny", 23.8, 26.8),
+    ("single", [(Q80, 896, 4864)], 333, "skinny", 19.4, 23.0),
+    ("single", [(Q80, 6144, 16384)], 96, "tiled", 83.7, 64.2),
+    ("single", [(Q4K, 14336, 4096)], 128, "tiled", 48.8, 33.7),
     ("swiglu", [(Q6K, 18944, 3584)], 96, "tiled", 99.9, 69.0),
     ("swiglu", [(Q6K, 28672, 8192)], 33, "tiled", 203.7, 148.1),
     ("swiglu", [(Q4K, 5632, 2048)], 64, "skinny", 16.2, 19.9),
