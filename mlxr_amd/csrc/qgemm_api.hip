@@ -23,11 +23,11 @@ constexpr int kGemvMaxM = 4;
 // Whether the automatic path runs a call with M <= kGemvMaxM on the GEMV kernel.  The GEMV
 // stages all M rows of X per workgroup (M = 3, 4 as four rows), so long rows cost it LDS
 // and occupancy; the skinny MFMA kernel's time hardly depends on M.  Measured on MI355X
-// (µs, GEMV / skinny MFMA without a K split): Llama-3-8B down (4096 x 14336) at M = 3 and
-// 4: 22.1 / 21.3 and 24.9 / 21.8 (the skinny one splits K with a workspace: about 17.5);
-// gate (14336 x 4096) at M = 4 16.5 / 15.1 and at M = 3 14.5 / 14.9; Llama-3-70B down (8192
-// x 28672) at M = 2 51.2 / 38.9; 4096 x 4096 at M = 4 7.4 / 9.8; the Q6_K lm_head (128256 x
-// 4096) at M = 4 116 / 146.
+// (Q4_K, us, GEMV / skinny MFMA): 4096 x 14336 at M = 2, 3 and 4 12.0 / 12.8, 22.0 / 13.2 and 24.0 /
+// 12.3; 14336 x 4096 at M = 3 and 4 14.7 / 12.5 and 16.1 / 12.5; 8192 x 28672 at M = 2 48.6 / 39.8;
+// 1024 x 4096 at M = 4 4.4 / 5.4.  The skinny kernel is ahead a little beyond these lines too (4096 x
+// 4096 at M = 4 7.5 / 6.1, the Q6_K lm_head, 128256 x 4096, 119 / 107), but it rounds the weights to
+// 16 bits, where the GEMV multiplies their exact values: calls on the GEMV keep it.
 bool gemv_auto(int M, const mlxr::PackedLayout& L) {
   if (M <= 1) return true;
   if (M > kGemvMaxM) return false;
@@ -344,10 +344,8 @@ namespace {
 
 // Whether a grouped call at M <= kGemvMaxM keeps an item in a grouped GEMV launch: where the
 // automatic path would run it on the GEMV, and also where it would not unless the weight is
-// very large (N*K >= 128 Mi): sharing one launch beats a skinny launch of its own for the
-// others (measured on MI355X, µs, grouped GEMV / items the automatic path gives the skinny
-// kernel on it: Llama-3-70B q,k at M = 3 20.3 / 23.0, with v 26.5 / 23.9; gate/up at M = 3 /
-// 4 94.4 / 105.7 grouped, 90.1 / 91.3 each on the skinny kernel).
+// very large (N*K >= 128 Mi; Llama-3-70B gate/up at M = 3 / 4, us, grouped GEMV / skinny 94.4 / 90.1
+// and 105.7 / 91.3): the others share one launch and keep the exact weights.
 bool grouped_gemv(int M, const mlxr::RunArgs& a) {
   return mlxr::gemv_groupable(a) && (gemv_auto(M, a.L) || (long)a.L.N * (long)a.L.K < (128L << 20));
 }
