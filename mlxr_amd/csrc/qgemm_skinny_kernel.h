@@ -1,6 +1,8 @@
 // Skinny GEMM (batched decode, and larger M in blocks of 32 rows for narrow weights):
-// Y[M,N] = X[M,K] . W[N,K]^T (+ bias) on the 16x16x32 MFMA, every weight byte streamed from
-// HBM once per block of rows.
+// Y[M,N] = X[M,K] . W[N,K]^T (+ bias) on the 16x16x32 MFMA, the weights streamed once per block of
+// rows (memory traffic counted against weights and activations: 1.03-1.15 at M <= 32, 1.48 for [13]
+// x (2 x 28672) x 8192, whose half lines of a step are partly evicted before the next; two blocks
+// of rows, M = 64, 1.26-1.39).
 //
 // Each weight is dequantized once in registers (the routines of qgemm_wdequant.h, the ones
 // the prefill GEMM and mlxr_qgemm_dequant use) and the rows of X ride along in the MFMA: the
